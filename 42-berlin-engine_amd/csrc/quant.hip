@@ -30,7 +30,10 @@ __device__ __forceinline__ uint8_t f32_to_fp8(float v)
     if ((__float_as_uint(a) >> 23) == 0)
         ex = -127;                                            // subnormal: far below e = 0
     const int up = ex + 1;
-    if (up >= kFp8ThrE0 && up < kFp8ThrE0 + kFp8ThrN && a >= c_fp8_thr[up - kFp8ThrE0])
+    // a threshold lies at most 64 ulps below its power of two
+    // (host_fp8_thresholds), so the table is read for such values only
+    if ((__float_as_uint(a) & 0x7FFFFFu) >= 0x7FFFC0u && up >= kFp8ThrE0 && up < kFp8ThrE0 + kFp8ThrN &&
+        a >= c_fp8_thr[up - kFp8ThrE0])
         ex = up;                                              // log2f rounded up to an integer
     int e = ex + 7;
     e = e < 0 ? 0 : (e > 15 ? 15 : e);
@@ -42,6 +45,13 @@ __device__ __forceinline__ uint8_t f32_to_fp8(float v)
     return (uint8_t)(sign | ((uint32_t)e << 3) | (uint32_t)m);
 }
 
+
+// quant_f32_to_int8's code of one element (ops_quant.c:262-267)
+__device__ __forceinline__ int8_t f32_to_int8(float v, float inv)
+{
+    const int c = (int)roundf(v * inv);
+    return (int8_t)(c > 127 ? 127 : (c < -127 ? -127 : c));
+}
 
 // block-wide absmax of one row (256 threads)
 __device__ __forceinline__ float row_absmax(const float *x, int cols, float *red)
@@ -73,11 +83,8 @@ __global__ __launch_bounds__(256) void k_quant_rows_int8(int8_t *q, float *scale
     }
     if (threadIdx.x == 0)
         scales[row] = scale;
-    for (int i = threadIdx.x; i < cols; i += blockDim.x) {
-        int v = (int)roundf(xr[i] * inv);
-        v = v > 127 ? 127 : (v < -127 ? -127 : v);
-        q[row * cols + i] = (int8_t)v;
-    }
+    for (int i = threadIdx.x; i < cols; i += blockDim.x)
+        q[row * cols + i] = f32_to_int8(xr[i], inv);
 }
 
 __global__ __launch_bounds__(256) void k_quant_rows_fp8(uint8_t *q, float *scales, const float *x,
@@ -96,6 +103,75 @@ __global__ __launch_bounds__(256) void k_quant_rows_fp8(uint8_t *q, float *scale
         scales[row] = scale;
     for (int i = threadIdx.x; i < cols; i += blockDim.x)
         q[row * cols + i] = f32_to_fp8(xr[i] * inv);
+}
+
+// Both codecs on rows whose elements come four to an aligned word.  HBM bound
+// (4 bytes in, 1 out per element): a block keeps its row in registers between
+// the absmax and the codes, so the row is read once, by NV 16-byte loads per
+// thread that are all in flight together, and leaves as 4-byte stores; the
+// one-element loops above read it twice, a round trip per element.  A pass of
+// quantize + product: FP8 8192 x 4096 x 14336 616 -> 559 us, INT8 500 x 4096 x
+// 4096 29.3 -> 24.3 us (the product alone 22).
+template <bool FP8, int NV>
+__global__ __launch_bounds__(256) void k_quant_rows_vec(uint8_t *__restrict__ q, float *__restrict__ scales,
+                                                        const float *__restrict__ x, int cols)
+{
+    __shared__ float red[4];
+    const size_t row = blockIdx.x;
+    const float4 *xr = (const float4 *)(x + row * cols);
+    const int n4 = cols / 4;
+    float4 v[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = threadIdx.x + 256 * j;
+        v[j] = i < n4 ? xr[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; j++)
+        m = fmaxf(fmaxf(fmaxf(m, fabsf(v[j].x)), fmaxf(fabsf(v[j].y), fabsf(v[j].z))), fabsf(v[j].w));
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0)
+        red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    const float amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    float scale = 1.0f, inv = 1.0f;
+    if (amax > 0.0f) {
+        scale = amax / (FP8 ? 224.0f : 127.0f);
+        inv = FP8 ? 1.0f / scale : 127.0f / amax;
+    }
+    if (threadIdx.x == 0)
+        scales[row] = scale;
+    uint32_t *qr = (uint32_t *)(q + row * cols);
+    auto code = [&](float e) {
+        return FP8 ? (uint32_t)f32_to_fp8(e * inv) : (uint32_t)(uint8_t)f32_to_int8(e, inv);
+    };
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = threadIdx.x + 256 * j;
+        if (i < n4)
+            qr[i] = code(v[j].x) | code(v[j].y) << 8 | code(v[j].z) << 16 | code(v[j].w) << 24;
+    }
+}
+
+// Rows of up to 16384 elements (16 words per thread) in 16-byte words; longer,
+// odd or unaligned ones take the one-element kernels.
+template <bool FP8>
+static bool launch_quant_vec(uint8_t *q, float *scales, const float *x, int rows, int cols, hipStream_t s)
+{
+    const int nv = (cols / 4 + 255) / 256;
+    if (cols % 4 || nv > 16 || (uintptr_t)x % 16 || (uintptr_t)q % 4)
+        return false;
+    const dim3 g(rows), b(256);
+    if (nv <= 1)
+        hipLaunchKernelGGL((k_quant_rows_vec<FP8, 1>), g, b, 0, s, q, scales, x, cols);
+    else if (nv <= 4)
+        hipLaunchKernelGGL((k_quant_rows_vec<FP8, 4>), g, b, 0, s, q, scales, x, cols);
+    else if (nv <= 8)
+        hipLaunchKernelGGL((k_quant_rows_vec<FP8, 8>), g, b, 0, s, q, scales, x, cols);
+    else
+        hipLaunchKernelGGL((k_quant_rows_vec<FP8, 16>), g, b, 0, s, q, scales, x, cols);
+    return true;
 }
 
 __global__ void k_dequant_rows_int8(float *out, const int8_t *q, const float *scales, int cols,
@@ -167,7 +243,8 @@ extern "C" int be42_quant_rows_int8(int8_t *q, float *scales, const float *x, in
     BE42_CHECK(rows >= 0 && cols > 0, "be42_quant_rows_int8: bad shape %d x %d", rows, cols);
     if (rows == 0)
         return BE42_OK;
-    hipLaunchKernelGGL(k_quant_rows_int8, dim3(rows), dim3(256), 0, as_stream(stream), q, scales, x, cols);
+    if (!launch_quant_vec<false>((uint8_t *)q, scales, x, rows, cols, as_stream(stream)))
+        hipLaunchKernelGGL(k_quant_rows_int8, dim3(rows), dim3(256), 0, as_stream(stream), q, scales, x, cols);
     BE42_LAUNCH_CHECK();
     return BE42_OK;
 }
@@ -182,7 +259,8 @@ extern "C" int be42_quant_rows_fp8(uint8_t *q, float *scales, const float *x, in
         return rc;
     if (rows == 0)
         return BE42_OK;
-    hipLaunchKernelGGL(k_quant_rows_fp8, dim3(rows), dim3(256), 0, as_stream(stream), q, scales, x, cols);
+    if (!launch_quant_vec<true>(q, scales, x, rows, cols, as_stream(stream)))
+        hipLaunchKernelGGL(k_quant_rows_fp8, dim3(rows), dim3(256), 0, as_stream(stream), q, scales, x, cols);
     BE42_LAUNCH_CHECK();
     return BE42_OK;
 }

@@ -85,3 +85,29 @@ def test_dequant_rows_int8(be, orc):
     out = be.dequant_rows_int8(q, s).cpu().numpy()
     want = q.cpu().numpy().astype(np.float32) * s.cpu().numpy()[:, None]
     np.testing.assert_array_equal(out, want)
+
+
+@pytest.mark.parametrize("cols", [4, 1020, 1024, 1028, 4096, 4100, 8192, 8196, 16384, 16388, 4098])
+def test_quant_rows_vector_edges(be, orc, cols):
+    """Row lengths at the edges of the in-register kernel (one to sixteen
+    16-byte words per thread) and past them, an absmax in the last element, a
+    row of zeros, and a source or destination that is not aligned."""
+    rng = np.random.default_rng(cols)
+    x = rng.standard_normal((3, cols)).astype(np.float32)
+    x[0, -1] = 9.0
+    x[1] = 0.0
+    dev = torch.from_numpy(x).cuda()
+    odd = torch.empty(3 * cols + 1, device="cuda")[1:].view(3, cols)
+    odd.copy_(dev)
+    for src in (dev, odd):
+        for name, quant, want in (("be42_quant_rows_int8", be.quant_rows_int8, orc.quant_int8),
+                                  ("be42_quant_rows_fp8", be.quant_rows_fp8, orc.quant_fp8)):
+            q, s = quant(src)
+            q2 = torch.zeros(3 * cols + 1, dtype=torch.uint8, device="cuda")[1:]
+            s2 = torch.zeros(3, device="cuda")
+            be._call(name, be.p(q2), be.p(s2), be.p(src), 3, cols, be.stream())
+            for r in range(3):
+                codes, scale = want(x[r])
+                np.testing.assert_array_equal(q[r].cpu().numpy(), codes)
+                np.testing.assert_array_equal(q2.view(3, cols)[r].cpu().numpy().view(codes.dtype), codes)
+                assert s[r].item() == s2[r].item() == scale
