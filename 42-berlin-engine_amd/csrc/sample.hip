@@ -42,27 +42,27 @@ constexpr int kSampT = 1024;
 // values into registers first, then used in the same order as one at a
 // time): a loop that uses each value as it arrives waits a full memory
 // round trip per element, and one block walks a whole 128k-entry row.
-//   strided: i = t, t + kSampT, ... (thread t), f(i, v)
-template <int U, class Ld, class F>
+//   strided: i = t, t + NT, ... (thread t of NT), f(i, v)
+template <int U, int NT = kSampT, class Ld, class F>
 __device__ __forceinline__ void strided_batches(int n, Ld &&ld, F &&f)
 {
-    for (int i0 = threadIdx.x; i0 < n; i0 += U * kSampT) {
+    for (int i0 = threadIdx.x; i0 < n; i0 += U * NT) {
         decltype(ld(0)) v[U];
 #pragma unroll
         for (int j = 0; j < U; j++) {
-            const int i = i0 + j * kSampT;
+            const int i = i0 + j * NT;
             v[j] = ld(i < n ? i : i0);
         }
 #pragma unroll
         for (int j = 0; j < U; j++)
-            if (i0 + j * kSampT < n)
-                f(i0 + j * kSampT, v[j]);
+            if (i0 + j * NT < n)
+                f(i0 + j * NT, v[j]);
     }
 }
 //   wave:    entries c0 .. c1 - 1 of one wave, 64 a step (lane l: entry
 //            a + l, T(0) past c1), f(a, v) returns true (wave-uniform) to stop
-template <int U, class T, class F>
-__device__ __forceinline__ void wave_steps(const T *__restrict__ q, int c0, int c1, F &&f)
+template <int U, class T, class Ld, class F>
+__device__ __forceinline__ void wave_steps(Ld &&ld, int c0, int c1, F &&f)
 {
     const int lane = threadIdx.x & (kWave - 1);
     for (int a0 = c0; a0 < c1; a0 += kWave * U) {
@@ -70,7 +70,7 @@ __device__ __forceinline__ void wave_steps(const T *__restrict__ q, int c0, int 
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int i = a0 + kWave * u + lane;
-            v[u] = i < c1 ? q[i] : T(0);
+            v[u] = i < c1 ? ld(i) : T(0);
         }
 #pragma unroll
         for (int u = 0; u < U; u++)
@@ -79,12 +79,14 @@ __device__ __forceinline__ void wave_steps(const T *__restrict__ q, int c0, int 
     }
 }
 
-// the block's row split into one contiguous range per wave, whole steps of 64
-__device__ __forceinline__ void wave_range(int n, int &c0, int &c1)
+// the wave's number as a scalar, so that its ranges and loops are scalar too
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }
+
+// contiguous slice `part` of `parts` of a row, whole steps of `unit` entries
+__device__ __forceinline__ void slice_of(int n, int part, int parts, int unit, int &c0, int &c1)
 {
-    constexpr int NW = kSampT / kWave;
-    const int cw = (((n + NW - 1) / NW) + kWave - 1) & ~(kWave - 1);
-    c0 = min(n, (int)(threadIdx.x / kWave) * cw);
+    const int cw = ((n + parts - 1) / parts + unit - 1) / unit * unit;
+    c0 = min(n, part * cw);
     c1 = min(n, c0 + cw);
 }
 
@@ -148,11 +150,12 @@ __global__ __launch_bounds__(kSampT) void k_probs(float *__restrict__ p, const v
 __device__ int block_first_exceeding(const float *__restrict__ q, int lim, float thr, float *sh, int *found)
 {
     constexpr int NW = kSampT / kWave;
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    const int wave = wave_id(), lane = threadIdx.x & (kWave - 1);
     int c0, c1;
-    wave_range(lim, c0, c1);
+    slice_of(lim, wave, NW, kWave, c0, c1);
+    auto ld = [&](int i) { return q[i]; };
     float carry = 0.0f;
-    wave_steps<8>(q, c0, c1, [&](int, float v) {
+    wave_steps<8, float>(ld, c0, c1, [&](int, float v) {
         carry += lane63(wave_prefix_sum(v));
         return false;
     });
@@ -171,7 +174,7 @@ __device__ int block_first_exceeding(const float *__restrict__ q, int lim, float
     }
     __syncthreads();
     carry = sh[NW + wave];
-    wave_steps<8>(q, c0, c1, [&](int a, float v) {
+    wave_steps<8, float>(ld, c0, c1, [&](int a, float v) {
         const float ps = wave_prefix_sum(v);
         const unsigned long long m = __ballot(carry + ps > thr);
         if (m) {
@@ -199,12 +202,14 @@ __global__ __launch_bounds__(kSampT) void k_pick_temperature(int *__restrict__ o
         out[b] = i < 0 ? n - 1 : i;
 }
 
-// the bit fields of a probability's pattern the three passes resolve
-// (12, 12 and 8 bits: the first pass spreads over exponent and 4 mantissa
-// bits, so the atomic additions of one wave rarely meet in one bucket)
+// the bit fields of a probability's pattern the three passes resolve (12, 10
+// and 8 bits; bits 30 and 31 are clear in [0, 1], other patterns weigh
+// nothing): the first pass spreads over 7 exponent and 5 mantissa bits, so the
+// atomic additions of one wave rarely meet in one bucket, and a bucket is
+// 1/32 of a power of two wide
 constexpr int kSelPasses = 3;
-constexpr int kSelShift[kSelPasses] = {20, 8, 0};
-constexpr int kSelBits[kSelPasses] = {12, 12, 8};
+constexpr int kSelShift[kSelPasses] = {18, 8, 0};
+constexpr int kSelBits[kSelPasses] = {12, 10, 8};
 constexpr int kSelBins = 1 << 12;
 
 // p as 62-bit fixed point, floor(p * 2^62), from the bits of p in [0, 1]:
@@ -221,49 +226,125 @@ __device__ __forceinline__ unsigned long long fixp_bits(unsigned k)
 }
 __device__ __forceinline__ unsigned long long fixp(float p) { return fixp_bits(__float_as_uint(p)); }
 
-struct TopPShared {
-    unsigned long long hist[kSelBins];   // bucket sums of a pass
-    unsigned long long scan[kSampT];
+template <int BINS>
+struct SelShared {
+    unsigned long long hist[BINS];   // bucket sums of a pass
+    unsigned long long scan[kSampT / kWave];
     int isum[kSampT / kWave];
     unsigned long long total, above;
-    int pos, bin, idx;
+    int pos, idx;
 };
+using TopPShared = SelShared<kSelBins>;
 
-// Exclusive block scan of one value per thread (thread order).
-template <class T>
-__device__ __forceinline__ T block_excl_scan_t(T v, T *sh)
+__device__ __forceinline__ unsigned long long shfl_u64(unsigned long long v, int l)
 {
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int o = 1; o < kSampT; o <<= 1) {
-        const T a = threadIdx.x >= (unsigned)o ? sh[threadIdx.x - o] : T(0);
-        __syncthreads();
-        sh[threadIdx.x] += a;
-        __syncthreads();
-    }
-    const T incl = sh[threadIdx.x];
-    __syncthreads();
-    return incl - v;
+    return (unsigned long long)(unsigned)__shfl((int)(v >> 32), l, kWave) << 32 | (unsigned)__shfl((int)v, l, kWave);
+}
+__device__ __forceinline__ unsigned long long shfl_up_u64(unsigned long long v, int o)
+{
+    const unsigned lo = __shfl_up((unsigned)v, o, kWave), hi = __shfl_up((unsigned)(v >> 32), o, kWave);
+    return (unsigned long long)hi << 32 | lo;
 }
 
-// The entry of p[0 .. n) at which the running sum of fixp(p), taken in
-// descending order of p with equal values in ascending index order, first
-// exceeds T; -1 if none does.  *above: the running sum before that entry;
-// *all: the sum of every entry.  Called by the whole block.
-__device__ int weighted_select(const float *__restrict__ p, int n, unsigned long long T, TopPShared &S,
-                               unsigned long long *above, unsigned long long *all)
+// Exclusive block scan of one value per thread (thread order of NT); sh: one
+// word per wave.
+template <int NT>
+__device__ __forceinline__ unsigned long long block_excl_scan(unsigned long long v, unsigned long long *sh)
+{
+    const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
+    unsigned long long incl = v;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const unsigned long long a = shfl_up_u64(incl, o);
+        incl += lane >= o ? a : 0ull;
+    }
+    if (lane == kWave - 1)
+        sh[wave] = incl;
+    __syncthreads();
+    unsigned long long before = 0;
+#pragma unroll
+    for (int w = 0; w < NT / kWave; w++)
+        before += w < wave ? sh[w] : 0ull;
+    __syncthreads();
+    return before + incl - v;
+}
+
+// A pass's buckets in descending order: thread t holds those at descending
+// positions 4t .. 4t + 3 (h) and the sum of every bucket before them (ex); NT
+// threads hold at most 4 NT buckets.
+struct BinScan {
+    unsigned long long h[4], ex;
+};
+template <int NT, class Sh>
+__device__ __forceinline__ BinScan scan_bins(const unsigned long long *hist, int nb, Sh &S)
+{
+    BinScan r;
+    unsigned long long ts = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int d = 4 * (int)threadIdx.x + j;
+        r.h[j] = d < nb ? hist[nb - 1 - d] : 0ull;
+        ts += r.h[j];
+    }
+    r.ex = block_excl_scan<NT>(ts, S.scan);
+    if (threadIdx.x == NT - 1)
+        S.total = r.ex + ts;
+    return r;
+}
+
+// The descending position of the bucket in which base + the running sum first
+// exceeds T (INT32_MAX: none does), *above the sum before that bucket.  Called
+// by the whole block.
+template <class Sh>
+__device__ __forceinline__ int crossing_bin(const BinScan &r, unsigned long long base, unsigned long long T,
+                                            Sh &S, unsigned long long *above)
+{
+    if (threadIdx.x == 0)
+        S.pos = INT32_MAX;
+    __syncthreads();
+    unsigned long long acc = base + r.ex, hit_above = 0;
+    int hit = -1;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (hit < 0 && r.h[j] && acc + r.h[j] > T) {
+            hit = 4 * (int)threadIdx.x + j;
+            hit_above = acc;
+        }
+        acc += r.h[j];
+    }
+    if (hit >= 0)
+        atomicMin(&S.pos, hit);
+    __syncthreads();
+    const int pos = S.pos;
+    if (hit >= 0 && hit == pos)
+        S.above = hit_above;
+    __syncthreads();
+    *above = S.above;
+    __syncthreads();
+    return pos;
+}
+
+// The entry of a list of n probabilities (ld(i): the bits of the i-th, in
+// ascending index order) at which the running sum of fixp, taken in descending
+// order of value with equal values in list order, first exceeds T; -1 if none
+// does.  The passes before pass0 are done: `prefix` holds the bits they found
+// and `base` the sum of every entry above them.  *above: the running sum
+// before the entry; *all: the sum of every entry (from pass 0).  Called by the
+// whole block.
+template <int NT, class Ld, class Sh>
+__device__ int weighted_select(Ld &&ld, int n, unsigned long long T, Sh &S, int pass0, unsigned prefix,
+                               unsigned long long base, unsigned long long *above, unsigned long long *all)
 {
     const int tid = threadIdx.x;
-    unsigned prefix = 0, pmask = 0;
-    unsigned long long base = 0;   // the sum of the entries above the current bucket
-    for (int pass = 0; pass < kSelPasses; pass++) {
+    unsigned pmask = 0;
+    for (int pass = 0; pass < pass0; pass++)
+        pmask |= ((1u << kSelBits[pass]) - 1) << kSelShift[pass];
+    for (int pass = pass0; pass < kSelPasses; pass++) {
         const int shift = kSelShift[pass], nb = 1 << kSelBits[pass];
-        for (int i = tid; i < nb; i += kSampT)
+        for (int i = tid; i < nb; i += NT)
             S.hist[i] = 0ull;
-        if (tid == 0)
-            S.pos = INT32_MAX;
         __syncthreads();
-        strided_batches<16>(n, [&](int i) { return __float_as_uint(p[i]); }, [&](int, unsigned k) {
+        strided_batches<16, NT>(n, ld, [&](int, unsigned k) {
             if ((k & pmask) == prefix) {
                 const unsigned long long f = fixp_bits(k);
                 if (f)
@@ -271,57 +352,25 @@ __device__ int weighted_select(const float *__restrict__ p, int n, unsigned long
             }
         });
         __syncthreads();
-        // thread t takes the buckets at descending positions 4t .. 4t + 3
-        unsigned long long h[4], ts = 0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int d = 4 * tid + j;
-            h[j] = d < nb ? S.hist[nb - 1 - d] : 0ull;
-            ts += h[j];
-        }
-        const unsigned long long ex = block_excl_scan_t<unsigned long long>(ts, S.scan);
-        if (pass == 0 && tid == kSampT - 1)
-            S.total = ex + ts;
-        unsigned long long acc = base + ex;
-        int hit = -1;
-        unsigned long long hit_above = 0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (hit < 0 && h[j] && acc + h[j] > T) {
-                hit = 4 * tid + j;
-                hit_above = acc;
-            }
-            acc += h[j];
-        }
-        if (hit >= 0)
-            atomicMin(&S.pos, hit);
-        __syncthreads();
-        const int pos = S.pos;
-        if (hit >= 0 && hit == pos) {
-            S.bin = nb - 1 - pos;
-            S.above = hit_above;
-        }
-        __syncthreads();
+        const BinScan r = scan_bins<NT>(S.hist, nb, S);
+        const int pos = crossing_bin(r, base, T, S, &base);
         if (pass == 0)
             *all = S.total;
-        const int bin = S.bin;
-        base = S.above;
-        __syncthreads();   // S is rewritten by the next pass
         if (pos == INT32_MAX)
             return -1;
-        prefix |= (unsigned)bin << shift;
+        prefix |= (unsigned)(nb - 1 - pos) << shift;
         pmask |= (unsigned)(nb - 1) << shift;
     }
     // the crossing entry has the value whose bits are `prefix`; among the
-    // entries of that value (ascending index) it is the k-th
+    // entries of that value (list order) it is the k-th
     const unsigned long long fv = fixp(__uint_as_float(prefix));   // > 0: its bucket's sum is positive
     const unsigned long long k = (T - base) / fv;
-    const int wave = tid / kWave, lane = tid & (kWave - 1);
+    const int wave = wave_id(), lane = tid & (kWave - 1);
     int c0, c1;
-    wave_range(n, c0, c1);
-    auto match = [&](int a, float v) { return __ballot(a + lane < c1 && __float_as_uint(v) == prefix); };
+    slice_of(n, wave, NT / kWave, kWave, c0, c1);
+    auto match = [&](int a, unsigned v) { return __ballot(a + lane < c1 && v == prefix); };
     int cnt = 0;   // entries of that value in this wave's range
-    wave_steps<8>(p, c0, c1, [&](int a, float v) {
+    wave_steps<8, unsigned>(ld, c0, c1, [&](int a, unsigned v) {
         cnt += __popcll(match(a, v));
         return false;
     });
@@ -335,7 +384,7 @@ __device__ int weighted_select(const float *__restrict__ p, int n, unsigned long
         off += S.isum[w];
     if ((unsigned long long)off <= k && k < (unsigned long long)(off + cnt)) {
         int rem = (int)(k - (unsigned long long)off);
-        wave_steps<8>(p, c0, c1, [&](int a, float v) {
+        wave_steps<8, unsigned>(ld, c0, c1, [&](int a, unsigned v) {
             unsigned long long m = match(a, v);
             const int c = __popcll(m);
             if (rem < c) {
@@ -358,20 +407,21 @@ __device__ int weighted_select(const float *__restrict__ p, int n, unsigned long
 
 // The last entry in descending order: the smallest value, the largest index
 // among equal ones.
-__device__ int last_entry(const float *__restrict__ p, int n, TopPShared &S)
+template <int NT, class Sh>
+__device__ int last_entry(const float *__restrict__ p, int n, Sh &S)
 {
     const int tid = threadIdx.x;
     unsigned long long best = 0;   // (~key << 32 | index): the largest is the last entry
-    strided_batches<16>(n, [&](int i) { return __float_as_uint(p[i]); }, [&](int i, unsigned k) {
+    strided_batches<16, NT>(n, [&](int i) { return __float_as_uint(p[i]); }, [&](int i, unsigned k) {
         const unsigned long long c = ((unsigned long long)~k << 32) | (unsigned)i;
         best = c > best ? c : best;
     });
-    unsigned long long *words = S.scan;
+    unsigned long long *words = S.hist;
     words[tid] = best;
     __syncthreads();
     if (tid == 0) {
         unsigned long long t = 0;
-        for (int i = 0; i < kSampT; i++)
+        for (int i = 0; i < NT; i++)
             t = words[i] > t ? words[i] : t;
         S.idx = (int)(unsigned)t;
     }
@@ -381,32 +431,449 @@ __device__ int last_entry(const float *__restrict__ p, int n, TopPShared &S)
     return idx;
 }
 
-// probabilities p (one row per block): cut at top_p, then draw with u
+// top_p as a threshold on the fixed-point sums (which stay near 2^62: a
+// threshold of 2 or more is never exceeded)
+__device__ __forceinline__ unsigned long long cut_threshold(float top_p)
+{
+    return top_p >= 2.0f ? ~0ull : (top_p > 0.0f ? (unsigned long long)((double)top_p * 0x1p62) : 0ull);
+}
+// u * (the set's sum); non-decreasing in the sum
+__device__ __forceinline__ unsigned long long draw_threshold(float u, unsigned long long total)
+{
+    return u > 0.0f ? (unsigned long long)fmin((double)u * (double)total, 1.8e19) : 0ull;
+}
+
+// One block per row of probabilities p: the set runs through the first entry
+// whose running sum exceeds top_p; the pick is the first entry whose running
+// sum exceeds u times the set's sum, or the set's last entry when none does.
 __global__ __launch_bounds__(kSampT) void k_top_p(int *__restrict__ out, const float *__restrict__ p, int n,
                                                   float top_p, const float *__restrict__ u)
 {
     __shared__ TopPShared S;
     const float *pb = p + (size_t)blockIdx.x * n;
-    // the set: through the first entry whose running sum exceeds top_p
-    // (the sums stay near 2^62: a threshold of 2 or more is never exceeded)
-    const unsigned long long T1 =
-        top_p >= 2.0f ? ~0ull : (top_p > 0.0f ? (unsigned long long)((double)top_p * 0x1p62) : 0ull);
+    auto ld = [&](int i) { return __float_as_uint(pb[i]); };
     unsigned long long above, all;
-    const int c = weighted_select(pb, n, T1, S, &above, &all);
+    const int c = weighted_select<kSampT>(ld, n, cut_threshold(top_p), S, 0, 0u, 0ull, &above, &all);
     const unsigned long long total = c >= 0 ? above + fixp(pb[c]) : all;
-    // r = u * (the set's sum); the first entry whose running sum exceeds it,
-    // or the set's last entry when none does
-    const float uu = u[blockIdx.x];
-    const unsigned long long R = uu > 0.0f ? (unsigned long long)fmin((double)uu * (double)total, 1.8e19) : 0ull;
+    const unsigned long long R = draw_threshold(u[blockIdx.x], total);
     int pick = -1;
     if (R < total) {
         unsigned long long a2, all2;
-        pick = weighted_select(pb, n, R, S, &a2, &all2);
+        pick = weighted_select<kSampT>(ld, n, R, S, 0, 0u, 0ull, &a2, &all2);
     }
     if (pick < 0)
-        pick = c >= 0 ? c : last_entry(pb, n, S);
+        pick = c >= 0 ? c : last_entry<kSampT>(pb, n, S);
     if (threadIdx.x == 0)
         out[blockIdx.x] = pick;
+}
+
+// ---- long rows: a row over kSlices blocks --------------------------------------
+// Bound by latency (a 128k-entry row is 0.5 MB; the passes wait on loads,
+// barriers and each other).  One block walks such a row ten times, at a
+// fraction of what a CU can load, and leaves the other CUs idle; here each step
+// of the same computation is a launch of kSlices blocks per row, and after the
+// first pass only the few entries in the buckets of the two crossings are
+// looked at again (k_row_bins, k_row_gather, k_row_pick: 13, 5 and 16 us of the
+// 50 us of 8 rows of 128256).  The results are the same bits: the
+// maximum and the 62-bit sums do not depend on the order, and the sum of the
+// exponentials keeps k_probs's (block j sums, row by row of kSampT entries,
+// the 64 columns that wave j of k_probs's block sums).
+constexpr int kSlices = kSampT / kWave;
+static_assert(kSlices == 16, "one block per wave of k_probs");
+
+// The buckets that can hold the two crossing entries: at descending positions
+// `cut` (the set's last entry; INT32_MAX: the set is every entry) and lo .. hi
+// (the pick; lo > hi: the set's last entry).  The set's sum is known to within
+// the cut bucket, so the draw's threshold, which grows with it, lies between
+// those of the two ends.
+struct PickBins {
+    int cut, lo, hi, pad;
+    unsigned long long all, cut_above, lo_above;   // the row's sum, the sums before those buckets
+};
+
+// a row's scratch besides its probabilities
+struct alignas(16) RowScratch {
+    unsigned long long hist[kSelBins];
+    float pmax[kSlices], psum[kSlices];
+    int cnt[kSlices * kSlices];   // candidates found by each wave of each block
+    PickBins bins;
+};
+
+template <bool BF16>
+__device__ __forceinline__ float logit(const void *logits, size_t i)
+{
+    return BF16 ? bf16_to_f32(((const uint16_t *)logits)[i]) : ((const float *)logits)[i];
+}
+
+// the slices' maxima; clears the row's buckets for k_row_hist
+template <bool BF16>
+__global__ __launch_bounds__(kSampT) void k_row_max(RowScratch *__restrict__ rs, const void *__restrict__ logits, int n)
+{
+    __shared__ float red[kSampT / 64];
+    const int b = blockIdx.y, tid = threadIdx.x;
+    RowScratch &R = rs[b];
+    for (int i = blockIdx.x * (kSelBins / kSlices) + tid; i < (int)(blockIdx.x + 1) * (kSelBins / kSlices); i += kSampT)
+        R.hist[i] = 0ull;
+    int c0, c1;
+    slice_of(n, blockIdx.x, kSlices, kSampT, c0, c1);
+    float m = -INFINITY;
+    const size_t row = (size_t)b * n + c0;
+    strided_batches<8>(c1 - c0, [&](int i) { return logit<BF16>(logits, row + i); },
+                       [&](int, float v) { m = fmaxf(m, v); });
+    m = block_reduce(m, red, true);
+    if (tid == 0)
+        R.pmax[blockIdx.x] = m;
+}
+
+// e_i = expf((x_i - max) / temp) and the sum over this block's 64 columns: for
+// each column in ascending order, then over the columns as wave_sum does
+constexpr int kExpRows = 128;   // rows of kSampT entries per round
+template <bool BF16>
+__global__ __launch_bounds__(kSampT) void k_row_exp(float *__restrict__ p, RowScratch *__restrict__ rs,
+                                                    const void *__restrict__ logits, int n, float temp,
+                                                    bool max_from_first)
+{
+    __shared__ float e[kExpRows][kWave];
+    const int b = blockIdx.y, lane = threadIdx.x & (kWave - 1), wave = wave_id();
+    RowScratch &R = rs[b];
+    const size_t row = (size_t)b * n;
+    float m = max_from_first ? logit<BF16>(logits, row) : -1e9f;
+    for (int j = 0; j < kSlices; j++)
+        m = fmaxf(m, R.pmax[j]);
+    const int col = blockIdx.x * kWave + lane;
+    float s = 0.0f;
+    for (int r0 = 0; r0 * kSampT < n; r0 += kExpRows) {
+        constexpr int U = kExpRows / kSlices;
+        float v[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const int i = (r0 + wave + kSlices * j) * kSampT + col;
+            v[j] = logit<BF16>(logits, row + (i < n ? i : 0));
+        }
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const int r = wave + kSlices * j, i = (r0 + r) * kSampT + col;
+            if (i < n)
+                p[row + i] = e[r][lane] = expf(__fdiv_rn(v[j] - m, temp));
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int rows = min(kExpRows, (n - col + kSampT - 1) / kSampT - r0);
+#pragma unroll 16
+            for (int r = 0; r < rows; r++)
+                s += e[r][lane];
+        }
+        __syncthreads();
+    }
+    if (wave == 0) {
+        s = wave_sum(s);
+        if (lane == 0)
+            R.psum[blockIdx.x] = s;
+    }
+}
+
+__device__ __forceinline__ float row_sum(const RowScratch &R)
+{
+    float s = R.psum[0];
+    for (int w = 1; w < kSlices; w++)
+        s = s + R.psum[w];
+    return s;
+}
+
+// p_i = e_i / sum, and the first pass's bucket sums of the row
+__global__ __launch_bounds__(kSampT) void k_row_hist(float *__restrict__ p, RowScratch *__restrict__ rs, int n)
+{
+    __shared__ unsigned long long hist[kSelBins];
+    const int b = blockIdx.y;
+    RowScratch &R = rs[b];
+    for (int i = threadIdx.x; i < kSelBins; i += kSampT)
+        hist[i] = 0ull;
+    const float s = row_sum(R);
+    int c0, c1;
+    slice_of(n, blockIdx.x, kSlices, kSampT, c0, c1);
+    float *pb = p + (size_t)b * n + c0;
+    __syncthreads();
+    strided_batches<8>(c1 - c0, [&](int i) { return pb[i]; }, [&](int i, float v) {
+        const float q = __fdiv_rn(v, s);
+        pb[i] = q;
+        const unsigned k = __float_as_uint(q);
+        const unsigned long long f = fixp_bits(k);
+        if (f)
+            atomicAdd(&hist[(k >> kSelShift[0]) & (kSelBins - 1)], f);
+    });
+    __syncthreads();
+    for (int i = threadIdx.x; i < kSelBins; i += kSampT)
+        if (hist[i])
+            atomicAdd(&R.hist[i], hist[i]);
+}
+
+__global__ __launch_bounds__(kSampT) void k_row_bins(RowScratch *__restrict__ rs, float top_p,
+                                                     const float *__restrict__ u)
+{
+    __shared__ TopPShared S;
+    RowScratch &R = rs[blockIdx.x];
+    const float uu = u[blockIdx.x];
+    const BinScan r = scan_bins<kSampT>(R.hist, kSelBins, S);
+    __syncthreads();
+    PickBins q;
+    unsigned long long a;
+    q.all = S.total;
+    q.cut = crossing_bin(r, 0ull, cut_threshold(top_p), S, &q.cut_above);
+    unsigned long long least = q.all, most = q.all;
+    if (q.cut != INT32_MAX) {
+        if ((int)threadIdx.x == q.cut / 4)
+            S.total = q.cut_above + r.h[q.cut & 3];
+        __syncthreads();
+        least = q.cut_above;
+        most = S.total;
+    }
+    q.lo = crossing_bin(r, 0ull, draw_threshold(uu, least), S, &q.lo_above);
+    q.hi = min(crossing_bin(r, 0ull, draw_threshold(uu, most), S, &a), q.cut);
+    if (threadIdx.x == 0)
+        R.bins = q;
+}
+
+// Each wave lists the entries of those buckets in its slice, in ascending
+// order, as (bits << 32 | index) from the slice's own place in `cand` on.
+__global__ __launch_bounds__(kSampT) void k_row_gather(unsigned long long *__restrict__ cand,
+                                                       RowScratch *__restrict__ rs, const float *__restrict__ p,
+                                                       int n)
+{
+    const int b = blockIdx.y, lane = threadIdx.x & (kWave - 1);
+    RowScratch &R = rs[b];
+    const int cut = R.bins.cut, lo = R.bins.lo, hi = R.bins.hi;
+    const int part = blockIdx.x * kSlices + wave_id();
+    int c0, c1, cnt = 0;
+    slice_of(n, part, kSlices * kSlices, kWave, c0, c1);
+    const float *pb = p + (size_t)b * n;
+    unsigned long long *cb = cand + (size_t)b * n + c0;
+    wave_steps<8, unsigned>([&](int i) { return __float_as_uint(pb[i]); }, c0, c1, [&](int a, unsigned k) {
+        const int d = kSelBins - 1 - (int)(k >> kSelShift[0]);   // negative for patterns above 1
+        const bool in = a + lane < c1 && d >= 0 && (d == cut || (d >= lo && d <= hi));
+        const unsigned long long m = __ballot(in);
+        if (in)
+            cb[cnt + __popcll(m & ((1ull << lane) - 1))] = (unsigned long long)k << 32 | (unsigned)(a + lane);
+        cnt += __popcll(m);
+        return false;
+    });
+    if (lane == 0)
+        R.cnt[part] = cnt;
+}
+
+// The draw over the listed entries, one block per row: few enough for LDS, and
+// a small block, whose many barriers are cheap.  Where they are too many
+// (equal or nearly equal logits) the passes read the whole row instead.
+constexpr int kPickT = 512;
+constexpr int kCandMax = 4096;
+struct TopPPick : SelShared<1 << kSelBits[1]> {
+    alignas(16) int start[kSlices * kSlices];
+};
+static_assert((1 << kSelBits[1]) >= kPickT && (1 << kSelBits[1]) <= 4 * kPickT && kSelBits[2] <= kSelBits[1], "buckets of the later passes");
+__global__ __launch_bounds__(kPickT) void k_row_pick(int *__restrict__ out, const unsigned long long *__restrict__ cand,
+                                                     const RowScratch *__restrict__ rs, const float *__restrict__ p,
+                                                     int n, float top_p, const float *__restrict__ u)
+{
+    __shared__ unsigned bits[kCandMax], idx[kCandMax];
+    __shared__ TopPPick S;
+    constexpr int parts = kSlices * kSlices, NW = kPickT / kWave;
+    const int b = blockIdx.x, lane = threadIdx.x & (kWave - 1), wave = wave_id();
+    const RowScratch &R = rs[b];
+    const PickBins q = R.bins;
+    const float uu = u[b];
+    const float *pb = p + (size_t)b * n;
+    const unsigned long long *cb = cand + (size_t)b * n;
+    // the parts' places in the list; a wave copies parts wave, wave + NW, ...
+    int total = 0;
+    {
+        const int4 c = *(const int4 *)&R.cnt[4 * lane];
+        int v = c.x + c.y + c.z + c.w, incl = v;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int a = __shfl_up(incl, o, kWave);
+            incl += lane >= o ? a : 0;
+        }
+        total = __builtin_amdgcn_readlane(incl, kWave - 1);
+        if (wave == 0)
+            *(int4 *)&S.start[4 * lane] = make_int4(incl - v, incl - v + c.x, incl - v + c.x + c.y, incl - c.w);
+    }
+    __syncthreads();
+    const bool listed = total <= kCandMax;
+    if (listed)
+        for (int i0 = wave; i0 < parts; i0 += NW * 8) {
+            unsigned long long c[8];
+            int cnt[8], c0[8], c1;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                slice_of(n, i0 + NW * j, parts, kWave, c0[j], c1);
+                cnt[j] = R.cnt[i0 + NW * j];
+                c[j] = lane < cnt[j] ? cb[c0[j] + lane] : 0ull;
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int at = S.start[i0 + NW * j];
+                for (int i = lane; i < cnt[j]; i += kWave) {
+                    const unsigned long long e = i == lane ? c[j] : cb[c0[j] + i];
+                    bits[at + i] = (unsigned)(e >> 32);
+                    idx[at + i] = (unsigned)e;
+                }
+            }
+        }
+    __syncthreads();
+    auto prefix = [&](int pos) { return (unsigned)(kSelBins - 1 - pos) << kSelShift[0]; };
+    auto draw = [&](auto &&ld, int m) {
+        unsigned long long above, unused, set = q.all;
+        int c = -1;
+        if (q.cut != INT32_MAX) {
+            c = weighted_select<kPickT>(ld, m, cut_threshold(top_p), S, 1, prefix(q.cut), q.cut_above, &above, &unused);
+            if (c < 0)
+                return -1;
+            set = above + fixp_bits(ld(c));
+        }
+        const unsigned long long T = draw_threshold(uu, set);
+        if (T >= set)
+            return c;
+        // the pick's bucket among lo .. hi
+        int pos = q.lo;
+        unsigned long long base = q.lo_above;
+        for (; pos < q.hi; pos += kWave) {
+            const int d = min(pos + lane, q.hi);
+            const unsigned long long h = pos + lane <= q.hi ? R.hist[kSelBins - 1 - d] : 0ull;
+            unsigned long long incl = h;
+#pragma unroll
+            for (int o = 1; o < kWave; o <<= 1) {
+                const unsigned long long a = shfl_up_u64(incl, o);
+                incl += lane >= o ? a : 0ull;
+            }
+            const unsigned long long over = __ballot(h && base + incl > T);
+            if (over) {
+                const int l = __ffsll(over) - 1;
+                pos += l;
+                base += shfl_u64(incl - h, l);
+                break;
+            }
+            base += shfl_u64(incl, kWave - 1);
+        }
+        return weighted_select<kPickT>(ld, m, T, S, 1, prefix(pos), base, &above, &unused);
+    };
+    int pick;
+    if (listed) {
+        pick = draw([&](int i) { return bits[i]; }, total);
+        if (pick >= 0)
+            pick = (int)idx[pick];
+    } else {
+        pick = draw([&](int i) { return __float_as_uint(pb[i]); }, n);
+    }
+    if (pick < 0)   // no cut and the draw above every sum: the smallest entry
+        pick = last_entry<kPickT>(pb, n, S);
+    if (threadIdx.x == 0)
+        out[b] = pick;
+}
+
+// p_i = e_i / sum and, for the running sums of block_first_exceeding, the sum
+// of each step of 64 entries of each of its 16 ranges.
+__global__ __launch_bounds__(kSampT) void k_row_steps(float *__restrict__ p, const RowScratch *__restrict__ rs,
+                                                      float *__restrict__ steps, int n)
+{
+    const int b = blockIdx.y, lane = threadIdx.x & (kWave - 1), wave = wave_id();
+    const float s = row_sum(rs[b]);
+    int c0, c1;
+    slice_of(n, blockIdx.x, kSlices, kWave, c0, c1);
+    float *pb = p + (size_t)b * n;
+    const int per = (n + kWave - 1) / kWave + kSlices;   // steps of a row, the ranges' last ones short
+    float *sb = steps + (size_t)b * per;
+    for (int a = c0 + wave * kWave; a < c1; a += kSampT) {
+        const int i = a + lane;
+        float v = 0.0f;
+        if (i < c1)
+            pb[i] = v = __fdiv_rn(pb[i], s);
+        const float t = lane63(wave_prefix_sum(v));
+        if (lane == 0)
+            sb[a / kWave] = t;
+    }
+}
+
+// The temperature draw from the steps' sums: wave w carries its range's
+// running sum from step to step as block_first_exceeding does and looks into
+// the steps that can hold a crossing.  Their running sums differ from carry +
+// step by a few roundings only.
+__global__ __launch_bounds__(kSampT) void k_row_walk(int *__restrict__ out, const float *__restrict__ p,
+                                                     const float *__restrict__ steps, int n,
+                                                     const float *__restrict__ r)
+{
+    __shared__ float sh[kSlices];
+    __shared__ int found;
+    const int b = blockIdx.x, lane = threadIdx.x & (kWave - 1), wave = wave_id();
+    int c0, c1;
+    slice_of(n, wave, kSlices, kWave, c0, c1);
+    const float *pb = p + (size_t)b * n;
+    const int per = (n + kWave - 1) / kWave + kSlices;
+    const float *sb = steps + (size_t)b * per + c0 / kWave;
+    const int ns = (c1 - c0 + kWave - 1) / kWave;
+    const float thr = r[b];
+    // f(step, its sum): true to stop; 64 steps' sums are loaded at a time
+    auto walk = [&](auto &&f) {
+        for (int k0 = 0; k0 < ns; k0 += kWave) {
+            const float t = k0 + lane < ns ? sb[k0 + lane] : 0.0f;
+            const int m = min(kWave, ns - k0);
+            for (int k = 0; k < m; k++)
+                if (f(k0 + k, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t), k))))
+                    return;
+        }
+    };
+    float carry = 0.0f;
+    walk([&](int, float t) {
+        carry += t;
+        return false;
+    });
+    if (lane == 0)
+        sh[wave] = carry;
+    if (threadIdx.x == 0)
+        found = INT32_MAX;
+    __syncthreads();
+    carry = 0.0f;
+    for (int w = 0; w < wave; w++)
+        carry += sh[w];
+    walk([&](int k, float t) {
+        if (!(carry + t * 1.00001f < thr * 0.99999f)) {
+            const int a = c0 + k * kWave;
+            const float ps = wave_prefix_sum(a + lane < c1 ? pb[a + lane] : 0.0f);
+            const unsigned long long m = __ballot(carry + ps > thr);
+            if (m) {
+                if (lane == 0)
+                    atomicMin(&found, a + __ffsll(m) - 1);
+                return true;
+            }
+        }
+        carry += t;
+        return false;
+    });
+    __syncthreads();
+    if (threadIdx.x == 0)
+        out[b] = found == INT32_MAX ? n - 1 : found;
+}
+
+// Rows go over kSlices blocks where the rows alone leave CUs idle and are long
+// enough to pay for the launches: one block / kSlices blocks, top-p us a call,
+// 16384 entries: 50 / 39 (1 row), 51 / 64 (64 rows); 32768: 69 / 39, 75 / 69;
+// 65536: 116 / 41, 121 / 73; 128256: 183 / 44, 219 / 87 (204 / 50 at 8 rows);
+// temperature at 16384: 15 / 17, 32768: 26 / 17, 28.5 / 28.2, 128256: 89 / 30,
+// 103 / 57.  The gain shrinks with the rows: at most one row per 512 entries.
+static bool long_rows(int n, int batch) { return n >= 32768 && batch <= n / 512 && batch <= 65535; }
+
+// maxima and exponentials of the rows (long_rows): p = e, not yet divided
+static int row_exp_launch(float *p, RowScratch *rs, const void *logits, bool bf16, int n, int batch, float temp,
+                          bool max_first, hipStream_t s)
+{
+    const dim3 g(kSlices, batch), t(kSampT);
+    if (bf16) {
+        hipLaunchKernelGGL(k_row_max<true>, g, t, 0, s, rs, logits, n);
+        hipLaunchKernelGGL(k_row_exp<true>, g, t, 0, s, p, rs, logits, n, temp, max_first);
+    } else {
+        hipLaunchKernelGGL(k_row_max<false>, g, t, 0, s, rs, logits, n);
+        hipLaunchKernelGGL(k_row_exp<false>, g, t, 0, s, p, rs, logits, n, temp, max_first);
+    }
+    BE42_LAUNCH_CHECK();
+    return BE42_OK;
 }
 
 int probs_launch(float *p, const void *logits, bool bf16, int n, int batch, float temp, bool max_first,
@@ -431,6 +898,22 @@ extern "C" int be42_sample_temperature_dt(int *out, const void *logits, int logi
     BE42_CHECK(out && logits && r, "be42_sample_temperature: null pointer");
     BE42_CHECK(n > 0 && batch > 0, "be42_sample_temperature: n %d, batch %d", n, batch);
     hipStream_t s = as_stream(stream);
+    if (long_rows(n, batch)) {
+        const size_t rsb = sizeof(RowScratch) * (size_t)batch, pb = (size_t)n * batch * 4;
+        const size_t per = (size_t)(n + kWave - 1) / kWave + kSlices;
+        uint8_t *ws = (uint8_t *)workspace(rsb + pb + per * batch * 4, s);
+        if (!ws)
+            return BE42_ENOMEM;
+        RowScratch *rs = (RowScratch *)ws;
+        float *p = (float *)(ws + rsb), *steps = (float *)(ws + rsb + pb);
+        const int rc = row_exp_launch(p, rs, logits, logits_bf16 != 0, n, batch, temp, false, s);
+        if (rc)
+            return rc;
+        hipLaunchKernelGGL(k_row_steps, dim3(kSlices, batch), dim3(kSampT), 0, s, p, rs, steps, n);
+        hipLaunchKernelGGL(k_row_walk, dim3(batch), dim3(kSampT), 0, s, out, p, steps, n, r);
+        BE42_LAUNCH_CHECK();
+        return BE42_OK;
+    }
     float *p = (float *)workspace((size_t)n * batch * 4, s);
     if (!p)
         return BE42_ENOMEM;
@@ -454,6 +937,25 @@ extern "C" int be42_sample_top_p_dt(int *out, const void *logits, int logits_bf1
     BE42_CHECK(out && logits && u, "be42_sample_top_p: null pointer");
     BE42_CHECK(n > 0 && batch > 0, "be42_sample_top_p: n %d, batch %d", n, batch);
     hipStream_t s = as_stream(stream);
+    if (long_rows(n, batch)) {
+        const size_t rsb = sizeof(RowScratch) * (size_t)batch, cb = (size_t)n * batch * 8;
+        uint8_t *ws = (uint8_t *)workspace(rsb + cb + cb / 2, s);
+        if (!ws)
+            return BE42_ENOMEM;
+        RowScratch *rs = (RowScratch *)ws;
+        unsigned long long *cand = (unsigned long long *)(ws + rsb);
+        float *p = (float *)(ws + rsb + cb);
+        const int rc = row_exp_launch(p, rs, logits, logits_bf16 != 0, n, batch, temp, true, s);
+        if (rc)
+            return rc;
+        const dim3 g(kSlices, batch), t(kSampT);
+        hipLaunchKernelGGL(k_row_hist, g, t, 0, s, p, rs, n);
+        hipLaunchKernelGGL(k_row_bins, dim3(batch), t, 0, s, rs, top_p, u);
+        hipLaunchKernelGGL(k_row_gather, g, t, 0, s, cand, rs, p, n);
+        hipLaunchKernelGGL(k_row_pick, dim3(batch), dim3(kPickT), 0, s, out, cand, rs, p, n, top_p, u);
+        BE42_LAUNCH_CHECK();
+        return BE42_OK;
+    }
     float *p = (float *)workspace((size_t)n * batch * 4, s);
     if (!p)
         return BE42_ENOMEM;

@@ -198,3 +198,37 @@ def test_dropin_samplers(be, orc):
     # (a draw of exactly 1.0, one in 32768, exceeds no running sum: the last index)
     got = [dl.sample_temperature(C.byref(D.tensor(x, D.DTYPE_F32, 1, 300)), 1.0, C.byref(arena)) for _ in range(3)]
     assert all(g in (123, 299) for g in got) and 123 in got
+
+
+@pytest.mark.parametrize("n", [32768, 32769, 40001, 65535, 131073, 150016])
+@pytest.mark.parametrize("kind", ["spread", "masked", "flat", "equal", "peaked", "nan"])
+def test_rows_over_several_blocks(be, n, kind):
+    """Rows over several blocks (few rows) pick the entry that one block per
+    row picks (more than n / 512 rows): the same sums, bit for bit.  Lengths at
+    the edges of the slices; logits whose candidates fill one bucket, few, or
+    more than fit on chip; draws and cuts at the ends of their range."""
+    rng = np.random.default_rng(n)
+    B = n // 512 + 1
+    x = (rng.standard_normal((4, n)) * dict(spread=2.5, masked=3.0, flat=0.02, equal=0.0, peaked=2.0, nan=1.0)[kind]).astype(np.float32)
+    if kind == "masked":
+        x[:, 1::2] = -np.inf
+        x[1, : n - 3] = -np.inf
+    if kind == "peaked":
+        x[:, n // 3] = 30.0
+        x[2, n - 1] = 31.0
+    if kind == "nan":
+        x[0, 5] = np.nan
+        x[1] = np.nan
+        x[2] = -np.inf
+    few = torch.from_numpy(x).cuda()
+    many = few.repeat((B + 3) // 4, 1)[:B].contiguous()
+    for u in ([0.0, 1.0, 0.5, 0.999999], [0.25, 0.75, 0.1, 0.9], rng.uniform(0, 1, 4)):
+        ut = torch.tensor(np.asarray(u, np.float32)).cuda()
+        um = ut.repeat((B + 3) // 4)[:B].contiguous()
+        for dt in (torch.float32, torch.bfloat16):
+            a, m = few.to(dt), many.to(dt)
+            for top_p in (0.0, 0.3, 0.9, 1.0, 2.0):
+                got, want = be.sample_top_p(a, 0.8, top_p, ut), be.sample_top_p(m, 0.8, top_p, um)
+                assert torch.equal(got, want[:4]), (u, dt, top_p)
+            got, want = be.sample_temperature(a, 0.8, ut), be.sample_temperature(m, 0.8, um)
+            assert torch.equal(got, want[:4]), (u, dt)
