@@ -298,9 +298,53 @@ __device__ __forceinline__ void attn_scores(const be42_kv_pool &P, AttnShared<HD
     }
 }
 
+// B. one head's closed-form online softmax (file header): lane <-> page in
+// the order of the recurrence, sv its 16 scores of which the first nt count.
+// sv becomes the weights (0 past nt); returns their sum, in every lane.
+__device__ __forceinline__ float attn_weights_row(float (&sv)[kPg], int nt)
+{
+    float lm = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < kPg; t++)
+        if (t < nt)
+            lm = fmaxf(lm, sv[t]);
+    // running max before this page: exclusive prefix max over the lanes
+    float m = wave_shift_up1(wave_prefix_max(lm), -INFINITY);
+    // the token steps without branches: every step is computed and
+    // selected (tokens past the page's count keep their state), which
+    // does the same operations for the valid tokens as the reference's
+    // loop; per-token branches cost more than the arithmetic
+    float av[kPg], lprod = 1.0f;
+#pragma unroll
+    for (int t = 0; t < kPg; t++) {
+        const bool v = t < nt;
+        const float st = sv[t];
+        const float mprev = m;
+        const float mn = fmaxf(m, st);
+        const float ex = fast_expf_neg(mprev - mn);
+        const float at = mprev == -INFINITY ? 1.0f : ex;
+        const float e = fast_expf_neg(st - mn);
+        m = v ? mn : m;
+        sv[t] = e;
+        av[t] = v ? at : 1.0f;
+        lprod = v ? lprod * at : lprod;
+    }
+    // rescales of all later pages: exclusive suffix product over the lanes
+    float pr = wave_shift_down1(wave_suffix_prod(lprod), 1.0f);
+    float ls = 0.0f;
+#pragma unroll
+    for (int t = kPg - 1; t >= 0; t--) {
+        const bool v = t < nt;
+        const float w = sv[t] * pr;
+        sv[t] = v ? w : 0.0f;
+        ls = v ? ls + w : ls;
+        pr *= av[t];   // av = 1 past the count
+    }
+    return wave_sum_dpp(ls);
+}
+
 // B. weights: wave g <-> head g, lane <-> selection position p (slot
-// order[p], or p when order is NULL), the closed-form online softmax of the
-// file header over the selection order; l = sum w.
+// order[p], or p when order is NULL), over the selection order; l = sum w.
 template <int HD, int G, int WAVES>
 __device__ __forceinline__ void attn_weights(AttnShared<HD, G, WAVES> &S, int ns, const int *order)
 {
@@ -314,45 +358,11 @@ __device__ __forceinline__ void attn_weights(AttnShared<HD, G, WAVES> &S, int ns
 #pragma unroll
         for (int t = 0; t < kPg; t++)
             sv[t] = s[slot * 17 + t];
-        float lm = -INFINITY;
+        const float ls = attn_weights_row(sv, nt);
 #pragma unroll
         for (int t = 0; t < kPg; t++)
             if (t < nt)
-                lm = fmaxf(lm, sv[t]);
-        // running max before this slot: exclusive prefix max over the lanes
-        float m = wave_shift_up1(wave_prefix_max(lm), -INFINITY);
-        // the token steps without branches: every step is computed and
-        // selected (tokens past the page's count keep their state), which
-        // does the same operations for the valid tokens as the reference's
-        // loop; per-token branches cost more than the arithmetic
-        float av[kPg], lprod = 1.0f;
-#pragma unroll
-        for (int t = 0; t < kPg; t++) {
-            const bool v = t < nt;
-            const float st = sv[t];
-            const float mprev = m;
-            const float mn = fmaxf(m, st);
-            const float ex = fast_expf(mprev - mn);
-            const float at = mprev == -INFINITY ? 1.0f : ex;
-            const float e = fast_expf(st - mn);
-            m = v ? mn : m;
-            sv[t] = v ? e : st;
-            av[t] = v ? at : 1.0f;
-            lprod = v ? lprod * at : lprod;
-        }
-        // rescales of all later slots: exclusive suffix product over the lanes
-        float pr = wave_shift_down1(wave_suffix_prod(lprod), 1.0f);
-        float ls = 0.0f;
-#pragma unroll
-        for (int t = kPg - 1; t >= 0; t--) {
-            const bool v = t < nt;
-            const float w = sv[t] * pr;
-            if (v)
-                s[slot * 17 + t] = w;
-            ls = v ? ls + w : ls;
-            pr *= av[t];   // av = 1 past the count
-        }
-        ls = wave_sum_dpp(ls);
+                s[slot * 17 + t] = sv[t];
         if (lane == 0)
             S.lsh[g] = ls;
     }

@@ -186,6 +186,12 @@ __device__ __forceinline__ float fast_expf(float x)
     return __int_as_float((int)__fmaf_rn(12102203.0f, x, 1065353216.0f));
 }
 
+// fast_expf of an argument that is not above zero (or NaN)
+__device__ __forceinline__ float fast_expf_neg(float x)
+{
+    return x < -87.0f ? 0.0f : __int_as_float((int)__fmaf_rn(12102203.0f, x, 1065353216.0f));
+}
+
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
 // round-to-nearest-even on the upper half, without a NaN case

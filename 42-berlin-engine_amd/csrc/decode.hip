@@ -2078,8 +2078,9 @@ static int prefill_pass(be42_decoder *d, int seq, int T, int p0, const AppendRun
         BE42_LAUNCH_CHECK();
         // the pass's K/V rows and the pages they fill: one launch each
         DEC_TRY(launch_append_run(*d->pool, runs[l], d->pmeta + list_off[l], d->pk, d->pv, st));
-        DEC_TRY(lsh_attention_prefix(*d->pool, d->pq, d->pmeta + (size_t)(2 + l) * T, lim, T, H, c.sparse_k,
-                                     c.cand_cap, scale, d->patt, d->psel, d->pnsel, d->psel_stride, st));
+        DEC_TRY(lsh_attention_prefix(*d->pool, d->pq, l * c.max_batch + seq, p0, d->pmeta + (size_t)(2 + l) * T, lim,
+                                     T, H, c.sparse_k, c.cand_cap, scale, d->patt, d->psel, d->pnsel, d->psel_stride,
+                                     st));
         DEC_TRY(xdig_prepare(d->pdig, d->patt, qd, T, fp8 != 0, st));
         DEC_TRY(pgemm(d, d->pxb, L.wo, L.so, dim, qd, T, st));
         BE42_HIP(norm(L.ffn_norm, d->pxb));                 // x += attention output

@@ -250,3 +250,36 @@ def test_prefill_fp8_forced_kv_against_oracle(be, orc, splits):
             break
         cur = g
     dec.close()
+
+
+@pytest.mark.parametrize("heads,n_kv,hd,n,splits,sparse_k", [
+    (4, 4, 128, 250, [1, 33, 34], 64), (8, 4, 128, 271, [5], 64), (6, 2, 128, 1045, None, 64), (16, 4, 128, 200, [7], 64),
+    (8, 8, 64, 1030, [700], 64), (16, 8, 64, 97, None, 64), (12, 4, 64, 300, [16, 48], 17), (32, 8, 64, 130, None, 7),
+])
+def test_prefill_dense_groups_bit_identical(be, orc, heads, n_kv, hd, n, splits, sparse_k):
+    """bf16 pages: the tokens that see at most sparse_k pages run 16 / G at a
+    time (from 768 token x KV-head pairs on).  Every group size and head dimension, passes that start and end
+    inside a page or a token group, and prompts that go on into routed tokens."""
+    rng, gc, wd, hpT = build(be, orc, "int8", OR_KV_BF16, sparse_k, 64, 1100, dims=(2, 256, heads, n_kv, hd, 256, 500))
+    prompt = rng.integers(0, gc["vocab"], n)
+    l1, s1, g1 = token_by_token(be, gc, wd, hpT, prompt, 4)
+    l2, s2, g2 = prefilled(be, gc, wd, hpT, prompt, 4, splits)
+    assert_same_cache(s1, s2)
+    np.testing.assert_array_equal(l1, l2)
+    assert g1 == g2
+
+
+def test_prefill_after_rewritten_positions(be, orc):
+    """Positions run again leave their page with the count of the last one
+    (the reference's append), and later tokens see that many of its tokens."""
+    rng, gc, wd, hpT = build(be, orc, "int8", OR_KV_BF16, 64, 64, 256, dims=(2, 256, 8, 8, 64, 256, 500))
+    runs = [(0, rng.integers(0, 500, 112)), (0, rng.integers(0, 500, 20)), (112, rng.integers(0, 500, 100))]
+    a, b = be42.Decoder(be, gc, wd, hpT), be42.Decoder(be, gc, wd, hpT)
+    la, lb = torch.empty((1, 500), device="cuda"), torch.empty(500, device="cuda")
+    for pos0, prompt in runs:
+        for i, t in enumerate(prompt):
+            a.step([int(t)], pos0 + i, logits=la)
+        b.prefill(prompt, pos0=pos0, logits=lb)
+        np.testing.assert_array_equal(la[0].cpu().numpy(), lb.cpu().numpy())
+    a.close()
+    b.close()
