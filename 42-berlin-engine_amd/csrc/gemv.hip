@@ -1089,6 +1089,198 @@ static void launch_dma(const GemvSegs &S, const uint8_t *dig, const float *sx, i
                        Kp, batch);
 }
 
+
+// GEMV straight from fp32 activations, one launch: small batches (the digit
+// columns fill one MFMA operand) of matrices whose every weight byte can be in
+// flight at once.  A block is 8 waves on TILES row tiles of 16 rows, wave w
+// taking its eighth of k (KU 128-byte steps) of all of them: its weights all go
+// to registers at the start (TILES * KU * 8 VGPRs, at most 64), and while they
+// stream the block forms the digit planes of x itself, in LDS.  Weights never
+// wait for the activations, and the digits cost no launch of their own (a
+// separate one takes ~3 us, and ~1.7 us pass before a launch that depends on
+// it).  Operands and epilogue are k_gemv's (32 consecutive bytes of a row per
+// lane and step for both types, the digits read at the same k), so INT8
+// results are the same bits.
+// Latency bound: 512 x 512 INT8 batch 1 5.7 -> 3.2 us a call, 4096 x 4096 8.9 ->
+// 6.9 us (2.4 TB/s), 8192 x 4096 14.0 -> 10.1 us (3.3 TB/s).
+constexpr int kDirectWaves = 8;
+constexpr int kDirectX = 5;                      // float4s of x per thread: batch * KU <= 10
+constexpr int direct_row(int ku) { return ku * 1024 + 16; }   // a digit column in LDS, padded against bank conflicts
+constexpr size_t direct_lds(int ku, int tiles, int cols)
+{
+    return (size_t)cols * direct_row(ku) + (size_t)kDirectWaves * tiles * 256 * 4;
+}
+
+template <bool FP8, int KU, int TILES>
+__global__ __launch_bounds__(kDirectWaves * 64) void k_gemv_direct(float *__restrict__ Y, const uint8_t *__restrict__ W,
+                                                                   const float *__restrict__ sw,
+                                                                   const float *__restrict__ x, int N, int K, int B)
+{
+    constexpr int ND = FP8 ? kF8Digits : kI8Digits;
+    constexpr int ROW = direct_row(KU), NT = kDirectWaves * 64;
+    using Tot = typename std::conditional<FP8, double, long long>::type;
+    using Acc = typename std::conditional<FP8, v4f, v4i>::type;
+    using Raw = typename std::conditional<FP8, float, int>::type;
+    extern __shared__ __align__(16) uint8_t dlds[];
+    __shared__ unsigned amax[16];
+    __shared__ float sxs[16];
+    uint8_t *dig = dlds;
+    Raw *part = (Raw *)(dlds + (size_t)B * ND * ROW);
+
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int r = lane & 15, g = lane >> 4;
+    if (tid < 16)
+        amax[tid] = 0u;
+    // x first: float4 i of the KU * 256 of each row (zero past K); the row is
+    // uniform over a wave
+    const int total4 = B * KU * 256;
+    float4 xv[kDirectX];
+#pragma unroll
+    for (int j = 0; j < kDirectX; j++) {
+        const int i0 = wave * 64 + NT * j;
+        xv[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (i0 < total4) {
+            const int b = i0 / (KU * 256), k = 4 * (i0 - b * KU * 256 + lane);
+            if (k < K)
+                xv[j] = *(const float4 *)(x + (size_t)b * K + k);
+        }
+    }
+    // then every weight byte of this block
+    v4i w[TILES][KU][2];
+    const int kb = wave * KU * 128 + 32 * g, klast = K - 16;
+#pragma unroll
+    for (int t = 0; t < TILES; t++) {
+        const int row = min((int)(blockIdx.x * TILES + t) * 16 + r, N - 1);
+        const uint8_t *wr = W + (size_t)row * K;
+#pragma unroll
+        for (int s = 0; s < KU; s++) {
+            w[t][s][0] = __builtin_nontemporal_load((const v4i *)(wr + min(kb + 128 * s, klast)));
+            w[t][s][1] = __builtin_nontemporal_load((const v4i *)(wr + min(kb + 128 * s + 16, klast)));
+        }
+    }
+    asm volatile("" ::: "memory");
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < kDirectX; j++) {
+        const int i0 = wave * 64 + NT * j;
+        if (i0 < total4) {
+            const float m = wave_prefix_max(
+                fmaxf(fmaxf(fabsf(xv[j].x), fabsf(xv[j].y)), fmaxf(fabsf(xv[j].z), fabsf(xv[j].w))));
+            if (lane == kWave - 1)
+                atomicMax(&amax[i0 / (KU * 256)], __float_as_uint(m));
+        }
+    }
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < kDirectX; j++) {
+        const int i0 = wave * 64 + NT * j;
+        if (i0 < total4) {
+            const int b = i0 / (KU * 256), c = i0 - b * KU * 256 + lane;
+            const float s = digit_scale<FP8>(__uint_as_float(amax[b]));
+            if (c == 0)
+                sxs[b] = s;
+            const float xe[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+            uint32_t word[ND];
+            digit_words<FP8>(xe, s, word);
+#pragma unroll
+            for (int d = 0; d < ND; d++)
+                *(uint32_t *)(dig + (b * ND + d) * ROW + 4 * c) = word[d];
+        }
+    }
+    lds_barrier();
+    // column c of the B operand: digit c % ND of batch row c / ND
+    const uint8_t *xcol = dig + (r < B * ND ? r : 0) * ROW + kb;
+    Acc acc[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; t++)
+        acc[t] = Acc{0, 0, 0, 0};
+#pragma unroll
+    for (int t = 0; t < TILES; t++)
+#pragma unroll
+        for (int s = 0; s < KU; s++) {
+            const v4i x0 = *(const v4i *)(xcol + 128 * s), x1 = *(const v4i *)(xcol + 128 * s + 16);
+            if constexpr (FP8) {
+                const v8i a = __builtin_shufflevector(w[t][s][0], w[t][s][1], 0, 1, 2, 3, 4, 5, 6, 7);
+                const v8i b = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
+                acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc[t], 0, 0, 0, 127, 0, 127);
+            } else {
+                acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[t][s][0], x0, acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[t][s][1], x1, acc[t], 0, 0, 0);
+            }
+        }
+#pragma unroll
+    for (int t = 0; t < TILES; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            part[((wave * TILES + t) * 16 + 4 * g + j) * 16 + r] = acc[t][j];
+    lds_barrier();
+    const double sxw = FP8 ? 1.0 : 1.0 / (double)(kI8Base * kI8Base);
+    for (int o = tid; o < TILES * 16 * B; o += NT) {
+        const int lr = o % (TILES * 16), b = o / (TILES * 16), row = blockIdx.x * TILES * 16 + lr;
+        if (row >= N)
+            continue;
+        Tot tot = 0;
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            Tot dsum = 0;
+#pragma unroll
+            for (int sl = 0; sl < kDirectWaves; sl++)
+                dsum += (Tot)part[(sl * TILES * 16 + lr) * 16 + b * ND + d];
+            if constexpr (FP8)
+                tot = tot + dsum * kF8Weight[d];
+            else
+                tot = tot + dsum * (Tot)(d == 0 ? kI8Base * kI8Base : (d == 1 ? kI8Base : 1));
+        }
+        Y[(size_t)b * N + row] = (float)((double)tot * ((double)sxs[b] * sxw * (double)sw[row]));
+    }
+}
+
+template <bool FP8, int KU, int TILES>
+static int launch_direct(float *y, const uint8_t *w, const float *sw, const float *x, int n, int k, int batch,
+                         hipStream_t s)
+{
+    const size_t lds = direct_lds(KU, TILES, batch * (FP8 ? kF8Digits : kI8Digits));
+    if (lds > 48 * 1024)
+        BE42_HIP(hipFuncSetAttribute((const void *)k_gemv_direct<FP8, KU, TILES>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const int blocks = ((n + 15) / 16 + TILES - 1) / TILES;
+    hipLaunchKernelGGL((k_gemv_direct<FP8, KU, TILES>), dim3(blocks), dim3(kDirectWaves * 64), lds, s, y, w, sw, x, n,
+                       k, batch);
+    BE42_LAUNCH_CHECK();
+    return BE42_OK;
+}
+
+// Whether (n, k, batch) runs as one k_gemv_direct launch; *rc its result.  The
+// lines lie where forming the digits in every block costs what the launch
+// saves (~1.3 us per 4096 elements of x; us, two launches / one, HBM-resident
+// weights, INT8, FP8 alike): 512 x 512 batch 1 5.7 / 3.2, batch 4 6.2 / 4.2;
+// 3072 x 3072 batch 1 7.7 / 5.2, batch 2 7.8 / 6.1, batch 4 8.0 / 8.2; 4096 x
+// 4096 batch 1 8.9 / 6.9, batch 2 9.1 / 8.2, batch 4 9.3 / 10.9; 8192 x 4096
+// batch 1 14.0 / 10.1; 16384 x 2048 batch 1 12.2 / 8.5, batch 5 12.6 / 12.2;
+// and where a block's weights stop fitting in 64 registers (14336 x 4096 batch
+// 1 15.4 / 16.4; 3000 x 8000 batch 1, weights in the Infinity Cache, 11.1 /
+// 11.5).
+// Overlapping x and y need the digits formed before the first output.
+template <bool FP8>
+static bool gemv_direct(float *y, const uint8_t *w, const float *sw, const float *x, int n, int k, int batch,
+                        hipStream_t s, int *rc)
+{
+    int ku = (k + 1023) / 1024;
+    ku = ku <= 4 ? ku : 6;
+    const int tiles = ((n + 15) / 16 + 255) / 256;
+    const bool apart = x + (size_t)batch * k <= y || y + (size_t)batch * n <= x;
+    if (k > 6144 || batch * (FP8 ? kF8Digits : kI8Digits) > 16 || batch * ku > 2 * kDirectX || !apart ||
+        getenv("BE42_GEMV_TILE"))
+        return false;
+#define BE42_DIRECT(KU, T)                                                                                         \
+    if (ku == KU && tiles <= T)                                                                                    \
+        return *rc = launch_direct<FP8, KU, T>(y, w, sw, x, n, k, batch, s), true;
+    BE42_DIRECT(1, 1) BE42_DIRECT(1, 2) BE42_DIRECT(1, 4) BE42_DIRECT(2, 1) BE42_DIRECT(2, 2) BE42_DIRECT(2, 4)
+    BE42_DIRECT(3, 1) BE42_DIRECT(3, 2) BE42_DIRECT(4, 1) BE42_DIRECT(4, 2) BE42_DIRECT(6, 1)
+#undef BE42_DIRECT
+    return false;
+}
+
 // Generic path for shapes the MFMA path does not take (k % 16 != 0, unaligned
 // pointers, batch > 16): one block per output row, fp32 dot of the
 // dequantized row, reduction through LDS.
@@ -1427,10 +1619,13 @@ static int gemv_launch(float *y, const uint8_t *w, const float *sw, const float 
         BE42_LAUNCH_CHECK();
         return BE42_OK;
     }
+    int rc = BE42_OK;
+    if (gemv_direct<FP8>(y, w, sw, x, n, k, batch, s, &rc))
+        return rc;
     void *buf = workspace(xdig_bytes(k, batch, FP8), s);
     if (!buf)
         return BE42_ENOMEM;
-    int rc = xdig_prepare(buf, x, k, batch, FP8, s);
+    rc = xdig_prepare(buf, x, k, batch, FP8, s);
     if (rc)
         return rc;
     return prepared_launch<FP8>(y, w, sw, buf, n, k, batch, s);
@@ -1496,12 +1691,16 @@ extern "C" int be42_gemv_noalloc(float *y, const void *w, const float *w_scale, 
         BE42_LAUNCH_CHECK();
         return BE42_OK;
     }
+    int rc = BE42_OK;
+    if (fp8 ? gemv_direct<true>(y, wb, w_scale, x, n, k, batch, s, &rc)
+            : gemv_direct<false>(y, wb, w_scale, x, n, k, batch, s, &rc))
+        return rc;
     const size_t need = xdig_bytes(k, batch, fp8 != 0);
     BE42_CHECK(need <= kNoAllocScratchBytes,
                "be42_gemv_noalloc: k=%d at batch %d needs %zu bytes of digit planes, more than the %zu-byte scratch "
                "(use be42_gemv_%s)", k, batch, need, kNoAllocScratchBytes, fp8 ? "fp8" : "q8");
     void *buf = nullptr;
-    int rc = gemv_scratch(&buf);
+    rc = gemv_scratch(&buf);
     if (rc)
         return rc;
     rc = xdig_prepare(buf, x, k, batch, fp8 != 0, s);

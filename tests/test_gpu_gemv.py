@@ -280,3 +280,42 @@ def test_gemv_coop_segments(be, orc, monkeypatch, kind, b):
             y = y.cpu().numpy()
             _check(y, want)
             assert rel_err(y, want) <= (1e-5 if kind == "int8" else 1e-4)
+
+
+@pytest.mark.parametrize("kind", ["int8", "fp8"])
+@pytest.mark.parametrize("n,k,b", [
+    (1, 16, 1), (17, 1008, 4), (4096, 1024, 5), (16384, 1024, 3), (16385, 1040, 1), (15, 1040, 4), (4097, 2048, 5),
+    (16383, 2064, 1), (33, 2064, 3), (8192, 3072, 3), (8193, 3072, 1), (31, 3088, 2), (4112, 4096, 2), (64, 4112, 1),
+    (4096, 6144, 1), (50, 6160, 1), (100, 8192, 1), (4097, 8192, 1), (100, 8208, 1),
+])
+def test_gemv_one_launch(be, orc, kind, n, k, b):
+    """be42_gemv forms the digits inside one launch for small batches; at the
+    edges of its range (rows per block, 1024-k steps, batch) and past them it
+    equals the two-step GEMV: INT8 the same bits, FP8 up to the order of the
+    fp32 sums of a row (at most 64 of them: 64 * 2^-24).  A zero batch row,
+    outliers, and an output that overlays the input."""
+    rng = np.random.default_rng(n + k + b)
+    wq = rng.integers(-127, 128, (n, k), dtype=np.int8) if kind == "int8" else rng.integers(0, 0x7F, (n, k), dtype=np.uint8)
+    ws = rng.uniform(0.005, 0.02, n).astype(np.float32)
+    x = rng.standard_normal((b, k)).astype(np.float32)
+    x[-1, ::5] *= 50.0
+    if b > 1:
+        x[0] = 0.0
+    wt, st, xt = torch.from_numpy(wq).cuda(), torch.from_numpy(ws).cuda(), torch.from_numpy(x).cuda()
+    y = be.gemv(wt, st, xt, kind, out=torch.full((b, n), float("nan"), device="cuda")).cpu().numpy()
+    two = be.gemv_prepared(wt, st, be.gemv_prepare(xt, kind), b, kind, torch.empty((b, n), device="cuda")).cpu().numpy()
+    if kind == "int8":
+        np.testing.assert_array_equal(y, two)
+    else:
+        assert rel_err(y, two) <= 64 * 2.0 ** -24
+    _check(y, orc.gemv(wq, ws, x, kind))
+    assert not (b > 1 and y[0].any())
+    m = max(n, k) * b
+    both = torch.zeros(m, device="cuda")
+    both[: b * k] = xt.reshape(-1)
+    be.gemv(wt, st, both[: b * k].view(b, k), kind, out=both)
+    over = both[: b * n].view(b, n).cpu().numpy()
+    if kind == "int8":
+        np.testing.assert_array_equal(over, two)
+    else:
+        assert rel_err(over, two) <= 64 * 2.0 ** -24
