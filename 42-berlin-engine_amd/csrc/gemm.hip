@@ -166,25 +166,33 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm(float *__restrict__ Y, c
     }
 
     // epilogue: lane l holds rows 4*(l/16)+e of column l%16 of each tile
+    // (scales loaded at once, as in k_gemm_dma)
+    float sxv[TM][4], swv[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+        swv[j] = sw[min(n0 + wn * (TN * 16) + j * 16 + r, N - 1)];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            sxv[i][e] = sx[min(m0 + wm * (TM * 16) + i * 16 + 4 * g + e, M - 1)];
 #pragma unroll
     for (int j = 0; j < TN; j++) {
         const int n = n0 + wn * (TN * 16) + j * 16 + r;
         if (n >= N)
             continue;
-        const float swn = sw[n];
 #pragma unroll
         for (int i = 0; i < TM; i++) {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int m = m0 + wm * (TM * 16) + i * 16 + 4 * g + e;
-                if (m < M) {
-                    float v;
-                    if constexpr (FP8)
-                        v = acc[i][j][e];
-                    else
-                        v = (float)acc[i][j][e];
-                    Y[(size_t)m * N + n] = (v * sx[m]) * swn;
-                }
+                float v;
+                if constexpr (FP8)
+                    v = acc[i][j][e];
+                else
+                    v = (float)acc[i][j][e];
+                if (m < M)
+                    Y[(size_t)m * N + n] = (v * sxv[i][e]) * swv[j];
             }
         }
     }
@@ -227,9 +235,11 @@ __device__ __forceinline__ void sched_interleave()
 // instruction fills 1 KB = 8 rows, lane l writing LDS bytes [16l, 16l+16),
 // i.e. row l/8, slot l%8, so each lane fetches global chunk
 // dma_slot(row, l%8) and the 8 lanes of a row read one full 128-byte line.
-// NS stages are resident in a ring (see the main loop).  Within a stage the
-// LDS reads of step 1 are interleaved with the matrix-core instructions of
-// step 0, and those of the next stage's step 0 with step 1.  Workgroup ids
+// NS stages are resident in a ring (see the main loop).  With up to two waves
+// per SIMD, the LDS reads of a stage's step 1 are interleaved with the
+// matrix-core instructions of step 0, and those of the next stage's step 0
+// with step 1; with four (16 waves) the waves cover each other's reads and
+// keep one step's fragments.  Workgroup ids
 // are spread over the 8 XCDs round-robin by the hardware; they are remapped
 // so that each XCD walks a contiguous run of the grouped tile order.
 // K must be a multiple of 128 and M*K, N*K below 2^32 (32-bit offsets);
@@ -366,57 +376,93 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dma(float *__restrict__ 
         if (st < nk)
             issue(st);
     if (nk >= NS)
-        wait_vmcnt<(NS - 1) * DPW>();
+        stage_barrier<(NS - 1) * DPW>();
     else
-        wait_vmcnt<0>();
-    __syncthreads();
-    Frags F[2];
-    load(0, 0, F[0]);
-    for (int st = 0; st < nk; st++) {
-        const int buf = st % NS, nbuf = (st + 1) % NS;
-        // step 0: read step 1's fragments while the matrix cores run step 0
-        __builtin_amdgcn_sched_barrier(0);
-        load(buf, 1, F[1]);
-        mfma(F[0]);
-        interleave();
-        __builtin_amdgcn_sched_barrier(0);
-        // step 1: stage st+1 must have landed and every wave be done with
-        // stage st before its buffer takes stage st+NS; then read stage
-        // st+1's first fragments (past the last stage the read is of stale
-        // LDS and unused)
+        stage_barrier<0>();
+    // stage st + 1 must have landed and every wave be done with stage st
+    // before its buffer takes stage st + NS
+    auto next_stage = [&](int st) {
         if (st + 1 < nk) {
             if (st + NS - 1 < nk)
-                wait_vmcnt<(NS - 2) * DPW>();
+                stage_barrier<(NS - 2) * DPW>();
             else
-                wait_vmcnt<0>();
-            __syncthreads();
+                stage_barrier<0>();
             if (st + NS < nk)
                 issue(st + NS);
         }
-        load(nbuf, 0, F[0]);
-        mfma(F[1]);
-        interleave();
+    };
+    if constexpr (NW >= 16) {
+        // four waves per SIMD hide the LDS reads, and 128 registers hold one
+        // step's fragments only
+        // (the empty statements keep the compiler from moving the
+        // products of a step past the next step's reads, which would keep
+        // both steps' fragments and spill)
+        auto done = [&]() {
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    asm volatile("" : "+v"(acc[i][j])::"memory");
+        };
+        Frags F;
+        load(0, 0, F);
+        for (int st = 0; st < nk; st++) {
+            mfma(F);
+            done();
+            load(st % NS, 1, F);
+            next_stage(st);
+            mfma(F);
+            done();
+            load((st + 1) % NS, 0, F);
+        }
+    } else {
+        Frags F[2];
+        load(0, 0, F[0]);
+        for (int st = 0; st < nk; st++) {
+            const int buf = st % NS, nbuf = (st + 1) % NS;
+            // step 0: read step 1's fragments while the matrix cores run step 0
+            __builtin_amdgcn_sched_barrier(0);
+            load(buf, 1, F[1]);
+            mfma(F[0]);
+            interleave();
+            __builtin_amdgcn_sched_barrier(0);
+            // step 1: read stage st+1's first fragments (past the last stage
+            // the read is of stale LDS and unused)
+            next_stage(st);
+            load(nbuf, 0, F[0]);
+            mfma(F[1]);
+            interleave();
+        }
     }
 
+    // every scale of this lane's outputs at once (clamped, so without
+    // branches): a load inside the store loop waits, output after output, for
+    // the stores before it too
+    float swv[TN];
 #pragma unroll
-    for (int j = 0; j < TN; j++) {
-        const int n = n0 + wn * (TN * 32) + j * 32 + r;
-        if (n >= N)
-            continue;
-        const float swn = sw[n];
+    for (int j = 0; j < TN; j++)
+        swv[j] = sw[min(n0 + wn * (TN * 32) + j * 32 + r, N - 1)];
 #pragma unroll
-        for (int i = 0; i < TM; i++) {
+    for (int i = 0; i < TM; i++) {
+        float sxv[16];
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+            sxv[e] = sx[min(m0 + wm * (TM * 32) + i * 32 + 8 * (e >> 2) + 4 * h + (e & 3), M - 1)];
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const int n = n0 + wn * (TN * 32) + j * 32 + r;
+            if (n >= N)
+                continue;
 #pragma unroll
             for (int e = 0; e < 16; e++) {
                 const int m = m0 + wm * (TM * 32) + i * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
-                if (m < M) {
-                    float v;
-                    if constexpr (FP8)
-                        v = acc[i][j][e];
-                    else
-                        v = (float)acc[i][j][e];
-                    Y[(size_t)m * N + n] = (v * sx[m]) * swn;
-                }
+                float v;
+                if constexpr (FP8)
+                    v = acc[i][j][e];
+                else
+                    v = (float)acc[i][j][e];
+                if (m < M)
+                    Y[(size_t)m * N + n] = (v * sxv[e]) * swv[j];
             }
         }
     }
@@ -448,33 +494,56 @@ static void launch_gemm(float *Y, const uint8_t *X, const float *sx, const uint8
                        M, N, K, tn);
 }
 
-// Kernel and tile choice.  K a multiple of 128 (and operands under 4 GiB):
-// the direct-to-LDS kernel, at 256 x 256 when that grid alone fills the 256
-// CUs, at 64 x 128 (4 waves of 32 x 64, a 4-stage ring) when 128 x 128 tiles
-// would leave CUs idle (fewer than 256 tiles: M = 512 at N = 4096), else at
-// 128 x 128.  Otherwise the register-staged 16x16 kernel at 128 x 128 when
+// Kernel and tile choice.  K a multiple of 128 (and operands under 4 GiB): the
+// direct-to-LDS kernel, with the largest tile whose grid still fills the 256
+// CUs (t = tiles of that size; us INT8 / FP8, K 4096 unless given):
+//   256 x 256, 16 waves, 2 stages     t128 > 512: 8192 x 14336 468 / 426 (with 8
+//       waves of 128 x 64 492 / 443), 1000 x 14336 63 / 56 (128 x 128: 72 / 66)
+//   128 x 128, 4 waves, 2 stages, two workgroups a CU   256 < t128 <= 512: 2048
+//       x 4096 40 / 37 (256 x 256: 56 / 49), 500 x 14336 39 / 36
+//   128 x 128, 16 waves, 4 stages     t128 <= 256 and more than 256 tiles of 64
+//       x 128: 1000 x 4096 25 / 23 (4 waves 30 / 29), 700 x 4096 24 / 21 (34 / 32)
+//   64 x 128, 8 waves, 4 stages       64 x 64 tiles > 256: 500 x 4096 16.9 / 16.0
+//       (4 waves 19 / 18), 512 x 4096 x 14336 47 / 43 (51 / 46)
+//   64 x 64, 4 waves, 4 stages        below: 256 x 4096 13.4 / 12.4 (64 x 128:
+//       16.4 / 15.3), 17 x 4096 12.0 / 10.9
+// At most 64 tokens keep to 64-row tiles and at most 128 to 128-row ones, whose
+// rows they fill.  Otherwise the register-staged 16x16 kernel at 128 x 128 when
 // its grid holds two workgroups per CU, else 64 x 128.
-// BE42_GEMM_TILE = 1..5 forces one of the five (1, 2 and 5 only where K
-// allows; 5 is the 64 x 128 direct-to-LDS tile).
+// BE42_GEMM_TILE = 1, 2, 5, 6, 7 (where K allows) forces a direct-to-LDS tile:
+// 256 x 256, 128 x 128 of 4 waves, 64 x 128, 64 x 64, 128 x 128 of 16 waves;
+// 3 and 4 the register-staged ones.
 template <bool FP8>
 static void gemm_dispatch(float *Y, const uint8_t *X, const float *sx, const uint8_t *W, const float *sw, int M,
                           int N, int K, hipStream_t s)
 {
-    const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-    const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256);
+    auto tiles = [&](long bm, long bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     const bool dma = K % 128 == 0 && (size_t)M * K < (1ull << 32) && (size_t)N * K < (1ull << 32);
     const char *e = getenv("BE42_GEMM_TILE");
-    const int force = e ? atoi(e) : 0;
-    if (dma && (force == 1 || (!force && tiles256 >= 256)))
-        launch_gemm_dma<FP8, 256, 256, 2, 4, 2>(Y, X, sx, W, sw, M, N, K, s);
-    else if (dma && (force == 5 || (!force && tiles128 < 256)))
-        launch_gemm_dma<FP8, 64, 128, 2, 2, 4>(Y, X, sx, W, sw, M, N, K, s);
-    else if (dma && (force == 2 || !force))
-        launch_gemm_dma<FP8, 128, 128, 2, 2, 2>(Y, X, sx, W, sw, M, N, K, s);
-    else if (force == 3 || (!force && tiles128 >= 512))
-        launch_gemm<FP8, 128, 128, 2, 2>(Y, X, sx, W, sw, M, N, K, s);
-    else
-        launch_gemm<FP8, 64, 128, 2, 2>(Y, X, sx, W, sw, M, N, K, s);
+    int tile = e ? atoi(e) : 0;
+    if (!dma && tile != 3 && tile != 4)
+        tile = tiles(128, 128) >= 512 ? 3 : 4;
+    else if (tile < 1 || tile > 7) {
+        if (M <= 64)
+            tile = tiles(64, 64) <= 512 ? 6 : 5;
+        else if (tiles(64, 64) <= 256)
+            tile = 6;
+        else if (tiles(64, 128) <= 256)
+            tile = 5;
+        else if (tiles(128, 128) <= 256)
+            tile = 7;
+        else
+            tile = tiles(128, 128) <= 512 || M <= 128 ? 2 : 1;
+    }
+    switch (tile) {
+    case 1: launch_gemm_dma<FP8, 256, 256, 4, 4, 2>(Y, X, sx, W, sw, M, N, K, s); break;
+    case 2: launch_gemm_dma<FP8, 128, 128, 2, 2, 2>(Y, X, sx, W, sw, M, N, K, s); break;
+    case 5: launch_gemm_dma<FP8, 64, 128, 2, 4, 4>(Y, X, sx, W, sw, M, N, K, s); break;
+    case 6: launch_gemm_dma<FP8, 64, 64, 2, 2, 4>(Y, X, sx, W, sw, M, N, K, s); break;
+    case 7: launch_gemm_dma<FP8, 128, 128, 4, 4, 4>(Y, X, sx, W, sw, M, N, K, s); break;
+    case 3: launch_gemm<FP8, 128, 128, 2, 2>(Y, X, sx, W, sw, M, N, K, s); break;
+    default: launch_gemm<FP8, 64, 128, 2, 2>(Y, X, sx, W, sw, M, N, K, s); break;
+    }
 }
 
 // Prefill GEMM with fp32 activations: the decode GEMV's arithmetic for many
@@ -612,17 +681,22 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig(float *__restrict__ 
 
     // lane l holds tokens 4*(l/16)+e of feature column l%16 of every tile
     const double sxw = FP8 ? 1.0 : 1.0 / (double)(kI8Base * kI8Base);
+    float sxv[4], swv[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+        swv[j] = sw[min(n0 + wn * (TN * 16) + j * 16 + r, N - 1)];
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        sxv[e] = sx[min(m0 + wm * 16 + 4 * g + e, M - 1)];
 #pragma unroll
     for (int j = 0; j < TN; j++) {
         const int n = n0 + wn * (TN * 16) + j * 16 + r;
         if (n >= N)
             continue;
-        const double swn = (double)sw[n];
+        const double swn = (double)swv[j];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int m = m0 + wm * 16 + 4 * g + e;
-            if (m >= M)
-                continue;
             double tot;
             if constexpr (FP8) {
                 tot = 0.0;
@@ -634,7 +708,8 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig(float *__restrict__ 
                                      (long long)acc[1][j][e] * kI8Base + (long long)acc[2][j][e];
                 tot = (double)it;
             }
-            Y[(size_t)m * N + n] = (float)(tot * ((double)sx[m] * sxw * swn));
+            if (m < M)
+                Y[(size_t)m * N + n] = (float)(tot * ((double)sxv[e] * sxw * swn));
         }
     }
 }
@@ -779,10 +854,9 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig_dma(const DigSegs S,
         if (st < nk)
             issue(st);
     if (nk >= NS)
-        wait_vmcnt<(NS - 1) * DPW>();
+        stage_barrier<(NS - 1) * DPW>();
     else
-        wait_vmcnt<0>();
-    __syncthreads();
+        stage_barrier<0>();
     Frags F[2];
     load(0, 0, F[0]);
     for (int st = 0; st < nk; st++) {
@@ -794,10 +868,9 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig_dma(const DigSegs S,
         __builtin_amdgcn_sched_barrier(0);
         if (st + 1 < nk) {
             if (st + NS - 1 < nk)
-                wait_vmcnt<(NS - 2) * DPW>();
+                stage_barrier<(NS - 2) * DPW>();
             else
-                wait_vmcnt<0>();
-            __syncthreads();
+                stage_barrier<0>();
             if (st + NS < nk)
                 issue(st + NS);
         }
@@ -806,19 +879,25 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig_dma(const DigSegs S,
         interleave();
     }
 
-    // lane l holds tokens 8*(e/4) + 4*(l/32) + e%4 of feature column l%32
+    // lane l holds tokens 8*(e/4) + 4*(l/32) + e%4 of feature column l%32; the
+    // scales of its outputs are loaded at once, as in k_gemm_dma
     const double sxw = FP8 ? 1.0 : 1.0 / (double)(kI8Base * kI8Base);
+    float sxv[16], swv[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+        swv[j] = sw[min(n0 + wn * (TN * 32) + j * 32 + r, N - 1)];
+#pragma unroll
+    for (int e = 0; e < 16; e++)
+        sxv[e] = sx[min(m0 + wm * 32 + 8 * (e >> 2) + 4 * h + (e & 3), M - 1)];
 #pragma unroll
     for (int j = 0; j < TN; j++) {
         const int n = n0 + wn * (TN * 32) + j * 32 + r;
         if (n >= N)
             continue;
-        const double swn = (double)sw[n];
+        const double swn = (double)swv[j];
 #pragma unroll
         for (int e = 0; e < 16; e++) {
             const int m = m0 + wm * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
-            if (m >= M)
-                continue;
             double tot;
             if constexpr (FP8) {
                 tot = 0.0;
@@ -830,7 +909,8 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig_dma(const DigSegs S,
                                      (long long)acc[1][j][e] * kI8Base + (long long)acc[2][j][e];
                 tot = (double)it;
             }
-            Y[(size_t)m * N + n] = (float)(tot * ((double)sx[m] * sxw * swn));
+            if (m < M)
+                Y[(size_t)m * N + n] = (float)(tot * ((double)sxv[e] * sxw * swn));
         }
     }
 }

@@ -1410,7 +1410,9 @@ static TileCfg pick_tile(bool fp8, int nc, int n, int k, int batch)
     // FP8 batch 8 17.8 -> 15.7 us; 14336 x 4096 INT8 batch 16 19.6 ->
     // 17.5 us; with four planes FP8 batch 16 is 4 groups, and 14336 x 4096
     // runs 29.1 -> 26.7 us here instead of on the split slab kernel).
-    if (n > 32768 || (n > 8192 && nc < 3) || (n > 4096 && nc >= 2 && nc <= 4)) {
+    // INT8 at one column group past 4096 rows: 5120 x 3072 9.3 -> 7.8 us, 6144
+    // x 4096 10.9 -> 9.4 (FP8 stays: 7.5 against 8.4, 9.2 against 10.2).
+    if (n > 32768 || (n > 8192 && nc < 3) || (n > 4096 && nc >= 2 && nc <= 4) || (n > 4096 && !fp8 && nc == 1)) {
         const int steps = (int)(xdig_kp(k, fp8) / 128);
         if (steps % kCoopWaves == 0 && steps / kCoopWaves <= 4)
             return TileCfg{0, 6, 0, kCoopWaves, 0, 4, 1};

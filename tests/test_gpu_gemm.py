@@ -224,3 +224,32 @@ def test_gemm_f32_rejects_bad_shapes(be):
     s = torch.ones(16, device="cuda")
     with pytest.raises(be42.Be42Error, match="k % 16 == 0"):
         be.gemm_f32(torch.zeros((4, 24), device="cuda"), w, s, "int8")
+
+
+@pytest.mark.parametrize("kind", ["int8", "fp8"])
+@pytest.mark.parametrize("tile", ["1", "2", "5", "6", "7"])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 128), (300, 270, 256), (257, 513, 384), (64, 129, 640), (130, 65, 1152)])
+def test_gemm_rings_and_edges(be, orc, monkeypatch, kind, tile, m, n, k):
+    """Each direct-to-LDS tile with fewer, as many and more stages than its
+    ring holds, and rows and columns one past and one short of its tiles;
+    five times on one input with the same result (the ring's barriers leave no
+    read of a slot in flight when it is refilled)."""
+    rng = np.random.default_rng(m + n + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+    xq, sx = _gpu_quant(be, x, kind)
+    wq, sw = _gpu_quant(be, w, kind)
+    hx, hsx = orc.quantize_rows(x, kind)
+    hw, hsw = orc.quantize_rows(w, kind)
+    monkeypatch.setenv("BE42_GEMM_TILE", tile)
+    first = None
+    for _ in range(5):
+        y = be.gemm(xq, sx, wq, sw, kind, out=torch.full((m, n), float("nan"), device="cuda")).cpu().numpy()
+        if first is None:
+            first = y
+            if kind == "int8":
+                np.testing.assert_array_equal(y, _exact_int8(hx, hsx, hw, hsw))
+            else:
+                assert rel_err(y.astype(np.float64), _exact_fp8(orc, hx, hsx, hw, hsw)) <= 2e-4
+        else:
+            np.testing.assert_array_equal(y, first)
