@@ -728,7 +728,8 @@ static void launch_gemm_dig(float *Y, const uint8_t *dig, const float *sx, const
 // owns BT = 32 WGM tokens x BN = 32 TN WGN features; wave (wm, wn) holds,
 // for its 32 tokens, one 32x32 accumulator per digit plane and feature tile.
 // A stage's LDS rows: digit d of token row t at d * BT + t, then the BN
-// weight rows, 128 bytes each with chunks placed by dma_slot.  The epilogue
+// weight rows, 128 bytes each with chunks placed by dma_slot.  With 12 waves the
+// loop is k_gemm_dma's for 16.  The epilogue
 // is k_gemm_dig's: digits combined in registers, one fp64 scaling.
 // Up to three weight matrices that share the activations (q/k/v, gate/up):
 // feature tiles are numbered through the segments one after another
@@ -751,13 +752,13 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig_dma(const DigSegs S,
     constexpr int NW = WGM * WGN;
     constexpr int BT = 32 * WGM, BN = 32 * TN * WGN, XR = ND * BT, R = XR + BN;
     constexpr int SBYTES = R * 128;
-    constexpr int DPW = R / 8 / NW;
-    static_assert(R % (8 * NW) == 0, "stage loads must divide over the waves");
+    constexpr int LOADS = R / 8, DPW = (LOADS + NW - 1) / NW;   // 1 KB each; the last waves repeat the last one
+    static_assert(R % 8 == 0, "whole loads");
     static_assert(XR % 8 == 0, "a load instruction stays within the digit rows or the weight rows");
     using AccT = typename std::conditional<FP8, v16f, v16i>::type;
     extern __shared__ __align__(1024) uint8_t lds_dyn[];
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int b = blockIdx.x, nb = gridDim.x;
     const int per = nb / 8, rem = nb % 8, x = b % 8, i8 = b / 8;
     const int tile = (x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per) + i8;
@@ -778,7 +779,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig_dma(const DigSegs S,
     uint32_t src[DPW];
 #pragma unroll
     for (int j = 0; j < DPW; j++) {
-        const int row = (wave * DPW + j) * 8 + (lane >> 3);
+        const int row = min(wave * DPW + j, LOADS - 1) * 8 + (lane >> 3);
         const uint32_t off = dma_slot(row, lane & 7) * 16;
         if (row < XR) {
             const int d = row / BT, t = min(m0 + row % BT, M - 1);
@@ -788,12 +789,13 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig_dma(const DigSegs S,
         }
     }
     auto issue = [&](int st) {
-        uint8_t *base = lds_dyn + (st % NS) * SBYTES + wave * DPW * 1024;
+        uint8_t *base = lds_dyn + (st % NS) * SBYTES;
 #pragma unroll
         for (int j = 0; j < DPW; j++) {
-            const uint8_t *g = (wave * DPW + j) * 8 < XR ? dig : W;
+            const int l = min(wave * DPW + j, LOADS - 1);
+            const uint8_t *g = l * 8 < XR ? dig : W;
             __builtin_amdgcn_global_load_lds((const void *)(g + src[j] + (size_t)st * 128),
-                                             (lds_void *)(base + j * 1024), 16, 0, 0);
+                                             (lds_void *)(base + l * 1024), 16, 0, 0);
         }
         asm volatile("" ::: "memory");
     };
@@ -857,15 +859,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig_dma(const DigSegs S,
         stage_barrier<(NS - 1) * DPW>();
     else
         stage_barrier<0>();
-    Frags F[2];
-    load(0, 0, F[0]);
-    for (int st = 0; st < nk; st++) {
-        const int buf = st % NS, nbuf = (st + 1) % NS;
-        __builtin_amdgcn_sched_barrier(0);
-        load(buf, 1, F[1]);
-        mfma(F[0]);
-        interleave();
-        __builtin_amdgcn_sched_barrier(0);
+    auto next_stage = [&](int st) {
         if (st + 1 < nk) {
             if (st + NS - 1 < nk)
                 stage_barrier<(NS - 2) * DPW>();
@@ -874,9 +868,42 @@ __global__ __launch_bounds__(WGM *WGN * 64) void k_gemm_dig_dma(const DigSegs S,
             if (st + NS < nk)
                 issue(st + NS);
         }
-        load(nbuf, 0, F[0]);
-        mfma(F[1]);
-        interleave();
+    };
+    if constexpr (NW >= 12) {
+        // as in k_gemm_dma
+        auto done = [&]() {
+#pragma unroll
+            for (int i = 0; i < ND; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    asm volatile("" : "+v"(acc[i][j])::"memory");
+        };
+        Frags F;
+        load(0, 0, F);
+        for (int st = 0; st < nk; st++) {
+            mfma(F);
+            done();
+            load(st % NS, 1, F);
+            next_stage(st);
+            mfma(F);
+            done();
+            load((st + 1) % NS, 0, F);
+        }
+    } else {
+        Frags F[2];
+        load(0, 0, F[0]);
+        for (int st = 0; st < nk; st++) {
+            const int buf = st % NS, nbuf = (st + 1) % NS;
+            __builtin_amdgcn_sched_barrier(0);
+            load(buf, 1, F[1]);
+            mfma(F[0]);
+            interleave();
+            __builtin_amdgcn_sched_barrier(0);
+            next_stage(st);
+            load(nbuf, 0, F[0]);
+            mfma(F[1]);
+            interleave();
+        }
     }
 
     // lane l holds tokens 8*(e/4) + 4*(l/32) + e%4 of feature column l%32; the
@@ -936,6 +963,49 @@ static void launch_gemm_dig_dma(DigSegs S, const uint8_t *dig, const float *sx, 
     }
     hipLaunchKernelGGL((k_gemm_dig_dma<FP8, WGM, WGN, TN, NS>), dim3(tm * tn), dim3(WGM * WGN * 64), lds, s, S, dig,
                        sx, M, K, (int)xdig_kp(K, FP8), tm, tm * tn);
+}
+
+// The tile whose grid takes the least time: rounds of 256 workgroups (one per
+// CU: a stage ring of any of them takes most of its LDS) times the time of a
+// full round, us at K = 3072 (times scale with K alike):
+//   32 tokens x 128 features, 4 waves, 4 stages   16
+//   64 x 128, 8 waves, 3 stages                   27 FP8, 25 INT8
+//   64 x 192, 12 waves, 2 stages                  35, 31
+//   64 x 256, 8 waves of 32 x 64, 2 stages        44, 40
+// FP8, 64 x 256 alone / by this rule: q/k/v of 100 tokens (5120 x 3072) 36 / 16,
+// gate/up (16384 x 3072) of 100 tokens 39 / 31, of 300 75 / 65, of 1000 (which
+// keeps 64 x 256, four full rounds) 177, o (3072 x 3072) of 1000 tokens 41 / 38,
+// down (3072 x 8192) of 1000 98 / 88, q/k/v of 1000 78 / 68.
+// BE42_GEMM_DIG = 3 .. 6 forces 64 x 128, 32 x 128, 64 x 192, 64 x 256.
+template <bool FP8>
+static void gemm_dig_dispatch(const DigSegs &S, const uint8_t *dig, const float *sx, int M, int K, int force,
+                              hipStream_t s)
+{
+    struct Tile {
+        int id, bt, bn, round;
+    };
+    constexpr Tile tiles[] = {{4, 32, 128, 16}, {3, 64, 128, FP8 ? 27 : 25}, {5, 64, 192, FP8 ? 35 : 31},
+                              {6, 64, 256, FP8 ? 44 : 40}};
+    int id = force;
+    if (id < 3 || id > 6) {
+        long best = 0;
+        for (const Tile &t : tiles) {
+            long n = 0;
+            for (int i = 0; i < S.nseg; i++)
+                n += (S.n[i] + t.bn - 1) / t.bn;
+            const long cost = (n * ((M + t.bt - 1) / t.bt) + 255) / 256 * t.round;
+            if (!best || cost < best) {
+                best = cost;
+                id = t.id;
+            }
+        }
+    }
+    switch (id) {
+    case 3: launch_gemm_dig_dma<FP8, 2, 4, 1, 3>(S, dig, sx, M, K, s); break;
+    case 4: launch_gemm_dig_dma<FP8, 1, 4, 1, 4>(S, dig, sx, M, K, s); break;
+    case 5: launch_gemm_dig_dma<FP8, 2, 6, 1, 2>(S, dig, sx, M, K, s); break;
+    default: launch_gemm_dig_dma<FP8, 2, 4, 2, 2>(S, dig, sx, M, K, s); break;
+    }
 }
 
 }  // namespace be42
@@ -1021,21 +1091,7 @@ static int gemm_dig_run(bool fp8, const be42_gemv_seg *segs, int nseg, const voi
     const char *e = getenv("BE42_GEMM_DIG");
     const int force = e ? atoi(e) : 0;
     if (dma && force != 1) {
-        if (fp8) {
-            // 64 tokens x 256 features: each wave's 4 digit fragments and 2
-            // weight fragments feed 8 matrix instructions (with 128 features,
-            // 5 fragments fed 4, and the LDS reads bounded the loop: the 3B
-            // shapes 15-20% slower)
-            if (force == 3)
-                launch_gemm_dig_dma<true, 2, 2, 2, 2>(S, dig, sx, m, k, s);
-            else
-                launch_gemm_dig_dma<true, 2, 4, 2, 2>(S, dig, sx, m, k, s);
-        } else {
-            if (force == 3)
-                launch_gemm_dig_dma<false, 2, 2, 2, 3>(S, dig, sx, m, k, s);
-            else
-                launch_gemm_dig_dma<false, 2, 4, 2, 2>(S, dig, sx, m, k, s);
-        }
+        fp8 ? gemm_dig_dispatch<true>(S, dig, sx, m, k, force, s) : gemm_dig_dispatch<false>(S, dig, sx, m, k, force, s);
     } else {
         for (int i = 0; i < nseg; i++) {
             if (fp8)

@@ -253,3 +253,27 @@ def test_gemm_rings_and_edges(be, orc, monkeypatch, kind, tile, m, n, k):
                 assert rel_err(y.astype(np.float64), _exact_fp8(orc, hx, hsx, hw, hsw)) <= 2e-4
         else:
             np.testing.assert_array_equal(y, first)
+
+
+@pytest.mark.parametrize("kind", ["int8", "fp8"])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 128), (33, 129, 256), (65, 193, 384), (31, 257, 640), (130, 191, 1152)])
+def test_gemm_f32_every_tile(be, kind, m, n, k, monkeypatch):
+    """The digit-plane GEMM's direct-to-LDS tiles (BE42_GEMM_DIG 3 .. 6) give
+    the same bits, five times over, as the tile its rule picks: fewer, as many
+    and more stages than their rings hold, edges one past and one short of the
+    tiles.  The rule's result is checked against the GEMV row by row."""
+    rng = np.random.default_rng(m + n + k)
+    wq, sw = _weights(rng, n, k, kind, be)
+    xt = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).cuda()
+    monkeypatch.delenv("BE42_GEMM_DIG", raising=False)
+    want = be.gemm_f32(xt, wq, sw, kind)
+    rows = torch.cat([be.gemv(wq, sw, xt[r:r + 16].contiguous(), kind) for r in range(0, m, 16)])
+    if kind == "int8":
+        assert torch.equal(want, rows)
+    else:
+        assert rel_err(want.cpu().numpy(), rows.cpu().numpy()) <= 1e-4
+    for tile in ("3", "4", "5", "6"):
+        monkeypatch.setenv("BE42_GEMM_DIG", tile)
+        for _ in range(5):
+            y = be.gemm_f32(xt, wq, sw, kind, out=torch.full((m, n), float("nan"), device="cuda"))
+            assert torch.equal(y, want), tile
