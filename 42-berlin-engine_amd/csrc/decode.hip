@@ -422,28 +422,30 @@ __global__ __launch_bounds__(256) void k_rope_rows(float *__restrict__ q, float 
 // its own costs about as much again.  One launch per layer runs, after the
 // layer's attention: the o projection, the residual add and RMSNorm, gate/up
 // with SiLU*up, the down projection, then the next layer's residual add,
-// RMSNorm, q/k/v and its RoPE + K/V append + seal -- with a grid barrier
-// between dependent phases.  Every block is resident (one per CU), keeps its
-// own copy of the phase's activation digit planes in LDS (it computes them
-// from the fp32 vector itself), and streams its row tiles of the phase's
-// weights straight from HBM into MFMA operand registers.  A phase's input
-// vector is loaded first; half of the block's weight loads leave while the
-// other half of its waves compute the digit planes; the phase's row scales
-// and output addresses load with the vector, so that only the cross-wave sum
-// and the stores follow the last matrix instruction.  (Weight loads issued
-// before a barrier were measured to slow the barrier itself more than they
-// gained, and so was a barrier in which every block reads a packed array of
-// all the arrival flags.)
+// RMSNorm, q/k/v and its RoPE + K/V append + seal.  Every block is resident
+// (one per CU), keeps its own copy of the phase's activation digit planes in
+// LDS (it computes them from the fp32 vector itself), and streams its row
+// tiles of the phase's weights straight from HBM into MFMA operand registers.
 //
-// Coherence: the activations one block writes and another reads go through
-// device-scope (agent) atomic stores and loads, which act at the device's
-// coherence point, so the barrier needs no L2 write-back or invalidate: a
-// block waits for its own stores (vmcnt), publishes an arrival flag, block 0
-// gathers every flag and publishes a release flag.  Flags hold increasing
-// barrier numbers (a per-decoder launch counter times kFBars plus the
-// barrier index), so graph replays need no reset.  Every wait is bounded: a
-// barrier that does not complete within ~kFSpinMax polls sets an error flag
-// the host reports, and the launch runs on (its results are then invalid).
+// What bounds it: the chain of four dependent phases, each a vector that every
+// block contributes to and every block needs (with all weights in the Infinity
+// Cache the launch took 47.0 us instead of 48.4).  So a phase's outputs go to an
+// exchange buffer that held kFEmpty words before, and its readers read the
+// buffer until no word is empty: one trip out and one in, with no wait for the
+// stores, no arrival flags and no release flag (which took 2.2 - 2.6 us a phase,
+// and 1.8 for the vector after it).  Waves 0-3 read the vector and compute the
+// digit planes; waves 4-7 issue their weight loads of the phase as soon as the
+// first of these reads have left, so that weights stream while the block waits.
+// Norm weights and row scales are loaded before the vector.  3B layer (FP8, 100.8
+// MB) 48.4 -> 41.2 us, its step 2250 -> 2046; 4-layer INT8 step of 512 / 1408
+// floats 222 -> 191.
+//
+// Coherence: exchanged words go through device-scope (agent) stores and loads,
+// which act at the device's coherence point.  Each word stands for itself, so
+// nothing is ordered against anything else.  Launches empty the buffers that
+// the launch before them used.  Every wait is bounded: one that does not
+// complete within ~kFSpinMax polls sets an error flag the host reports, and the
+// launch runs on (its results are then invalid).
 //
 // Arithmetic: the row kernels' (RMSNorm sums of squares in the same thread
 // layout and tree, the same digit split and SiLU), and the GEMV's single
@@ -455,7 +457,6 @@ constexpr int kFW = kFT / kWave;          // waves per block
 constexpr int kFMaxU = 12;                // MFMA steps (128 k-bytes) one wave holds in registers
 constexpr int kFMaxTiles = 8;             // 16-row tiles of one block in one phase
 constexpr int kFDigBytes = 84 * 1024;     // LDS digit planes; also keeps one block per CU
-constexpr int kFBars = 8;                 // barrier numbers per launch
 constexpr unsigned kFSpinMax = 1u << 16;  // polls (about 1 us each) before a wait gives up
 
 __device__ __forceinline__ float ld_dev(const float *p)
@@ -470,20 +471,78 @@ __device__ __forceinline__ void st_dev(__attribute__((address_space(1))) float *
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Device-scope (sc1) direct-to-LDS loads of a vector other blocks wrote:
-// lane l of wave w moves floats 4 (64 w + l + 256 q) .. + 3 for q = 0, 1, ...
-// (threads < kRowT, n floats, n a multiple of 4) into dst at the same float
-// index.  The caller waits (vmcnt) before reading dst.
-__device__ __forceinline__ void vec_to_lds(const float *src, float *dst, int n)
+// Values exchanged inside a launch: the buffer holds kFEmpty words until their
+// values arrive; a value with those bits (a NaN) is stored as another NaN.
+constexpr uint32_t kFEmpty = 0xFFFFFFFFu;
+__device__ __forceinline__ float ex_value(float y)
 {
-    const int tid = threadIdx.x, wave = tid >> 6;
-    if (tid >= kRowT)
-        return;
-    for (int q = 0; (wave * 64 + q * kRowT) * 4 < n; q++) {
-        const int i4 = tid + q * kRowT;
-        if (4 * i4 < n)
-            __builtin_amdgcn_global_load_lds((const void *)(src + 4 * i4),
-                                             (lds_void *)(dst + 4 * (wave * 64 + q * kRowT)), 16, 0, 16);
+    return __float_as_uint(y) == kFEmpty ? __uint_as_float(0xFFFFFFFEu) : y;
+}
+// Block barrier for data in LDS only: loads in flight stay in flight.
+__device__ __forceinline__ void lds_barrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// How long a wait may last, and where one that gave up is reported.
+struct ExWait {
+    int *err;
+    unsigned spin_max;   // polls before a wait gives up
+    bool never;          // a test: no wait completes
+};
+// after `spins` polls of a wait: whether to give up (the bound is reached, or
+// another wait of the launch has given up)
+__device__ __forceinline__ bool ex_give_up(const ExWait &w, unsigned spins)
+{
+    if (spins > w.spin_max) {
+        atomicExch(w.err, 1);
+        return true;
+    }
+    return (spins & 255) == 0 && __hip_atomic_load(w.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+
+// A vector of n floats (a multiple of 4) into LDS, by waves 0-3: lane l of
+// wave w moves floats 4 (64 w + l + 256 q) .. + 3 for q = 0, 1, ... with
+// device-scope direct-to-LDS loads (aux 16: sc1) and reads back only those.
+// `issued` runs once, after the first loads have left.  ex: the vector is an
+// exchange buffer; the 64-lane chunks that still hold kFEmpty are read again.
+template <class Issued>
+__device__ __forceinline__ void vec_to_lds(const float *src, float *dst, int n, bool ex, const ExWait &wt,
+                                           Issued &&issued)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int left4 = n / 4 - wave * 64;                                  // this wave's first float4 to the end
+    const int nq = left4 > 0 ? (left4 + kRowT - 1) / kRowT : 0;           // its chunks
+    const float *sp = src + 4 * (wave * 64 + lane);
+    float *dw = dst + 4 * wave * 64;
+    unsigned pend = (1u << nq) - 1;
+    for (unsigned spins = 0;; spins++) {
+#pragma unroll 1
+        for (int q = 0; q < nq; q++)
+            if ((pend >> q & 1) && lane < left4 - q * kRowT)
+                __builtin_amdgcn_global_load_lds((const void *)(sp + 4 * q * kRowT), (lds_void *)(dw + 4 * q * kRowT),
+                                                 16, 0, 16);
+        if (spins == 0)
+            issued();
+        wait_vmcnt<0>();
+        asm volatile("" ::: "memory");
+        if (!ex)
+            return;
+        unsigned left = 0;
+#pragma unroll 2
+        for (int q = 0; q < nq; q++) {
+            bool empty = wt.never;
+            if (lane < left4 - q * kRowT) {
+                const uint4 u = *(const uint4 *)(dw + 4 * (lane + q * kRowT));
+                empty |= max(max(u.x, u.y), max(u.z, u.w)) == kFEmpty;
+            }
+            left |= __any(empty) ? 1u << q : 0u;
+        }
+        pend = left;
+        if (!pend || ex_give_up(wt, spins + 1))
+            return;
+        // the checks' LDS reads are done before the next loads land there
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
 }
 
@@ -507,9 +566,16 @@ struct EmbRow {
 };
 
 struct FusedArgs {
-    FPhase o, gu, down, qkv;      // qkv.nseg == 0: the last layer
+    FPhase ph[4];                 // o, gate/up, down, and the next layer's q/k/v
+    int last;                     // the launch's last phase (the last layer: 2)
     const float *att;
-    float *X, *Hb, *XB, *H2, *q, *k, *v;
+    const float *ex_o, *ex_dn, *ex_h2;      // exchanged in this launch: o's, down's and silu(gate) * up's outputs
+    float *ex_q, *ex_k, *ex_v;              // and q / k / v
+    float *clr[2];                          // exchange buffers to empty for later launches (none in use by this one)
+    int nclr[2];                            // floats of each
+    const float *X;                         // the layer's input
+    float *Xout;                            // the next layer's input; the last layer: its h = X + o
+    float *q, *k, *v;
     const uint16_t *ffn_norm, *attn_norm;   // this layer's FFN norm, the next layer's attention norm
     be42_kv_pool P;
     const AppendStepArgs *app;              // the next layer's append
@@ -517,70 +583,12 @@ struct FusedArgs {
     const int *pos_p;
     int rope_len, dim, hidden, qd, kd, H, KV;
     float eps;
-    unsigned *flags, *gen;
-    int *err;
-    unsigned spin_max;   // polls before a grid-barrier wait gives up
-    unsigned bias;       // added to the numbers waited for (0; a test sets it so no wait completes)
+    ExWait wait;
     float *att_out;      // the next layer's dense attention output (null: a launch of its own)
     float att_scale;
     EmbRow er;           // k_fused_layer<..., START>: the step's token, whose embedding is layer 0's input
     int pf_route;        // the next layer's attention routes: warm the L2 with its routing tables
 };
-
-struct GridBar {
-    unsigned *flags;
-    unsigned base;
-    int nb;
-    int *err;
-    unsigned spin_max, bias;
-};
-
-__device__ __forceinline__ bool flag_before(unsigned v, unsigned target) { return (int)(v - target) < 0; }
-
-// Arrive, run `during` (loads of the next phase's weights), then wait for
-// every block.  After a timed-out wait (error flag set) later barriers do not
-// wait again; whether to wait is decided once per block.
-template <class F>
-__device__ __forceinline__ void grid_barrier(const GridBar &gb, unsigned idx, F &&during)
-{
-    __shared__ int failed;
-    const unsigned target = gb.base + idx, awaited = target + gb.bias;
-    wait_vmcnt<0>();              // this thread's stores have completed
-    __syncthreads();
-    // arrive, then read the error word (its round trip overlaps the wait)
-    if (threadIdx.x == 0) {
-        __hip_atomic_store(gb.flags + blockIdx.x * 32, target, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        failed = __hip_atomic_load(gb.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-    }
-    during();
-    __syncthreads();
-    const bool skip = failed;
-    if (blockIdx.x == 0 && !skip) {
-        for (int i = threadIdx.x; i < gb.nb; i += blockDim.x) {
-            unsigned spins = 0;
-            while (flag_before(__hip_atomic_load(gb.flags + i * 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                               awaited))
-                if (++spins > gb.spin_max) {
-                    atomicExch(gb.err, 1);
-                    break;
-                }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0)
-            __hip_atomic_store(gb.flags + gb.nb * 32, target, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (threadIdx.x == 0 && !skip) {
-        unsigned spins = 0;
-        while (flag_before(__hip_atomic_load(gb.flags + gb.nb * 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                           awaited))
-            if (++spins > gb.spin_max) {
-                atomicExch(gb.err, 2);
-                break;
-            }
-    }
-    __syncthreads();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
 
 __device__ __forceinline__ int ph_count(const FPhase &ph, int b, int nb)
 {
@@ -798,13 +806,13 @@ __device__ __forceinline__ void ph_compute(const FPhase &ph, int b, int nb, cons
         if (ph.silu)
             ybuf[i] = y;
         else if (oo.y)
-            st_dev(oo.y, y);
+            st_dev(oo.y, ex_value(y));
     }
     if (ph.silu) {
         __syncthreads();
         if (oo.y) {
             const int p = i >> 4, r = i & 15;
-            st_dev(oo.y, silu_mul1(ybuf[2 * p * 16 + r], ybuf[(2 * p + 1) * 16 + r], !oo.tail));
+            st_dev(oo.y, ex_value(silu_mul1(ybuf[2 * p * 16 + r], ybuf[(2 * p + 1) * 16 + r], !oo.tail)));
         }
     }
 }
@@ -818,7 +826,7 @@ __device__ __forceinline__ float *dig_stage(uint8_t *dig, int nd, int K)
 // Waves 0-3 of a block wait for each other through an LDS counter (waves
 // 4-7 take no part: they may be stalled issuing weight loads, and a block
 // barrier would hold waves 0-3 behind them).  Every call adds 4 to the
-// target; the wait is bounded like the grid barrier's.
+// target; the wait is bounded like the exchange's.
 struct QuadSync {
     int *cnt;     // LDS, 0 at kernel start
     int target;
@@ -852,162 +860,135 @@ __device__ __forceinline__ float quad_max(float v, float *red, QuadSync &q)
     return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-// Digit planes of a vector written by other blocks (K a multiple of 128,
-// at most kRowT * 4 * kFVecG).  Waves 0-3 stage it in LDS with device-scope
-// loads; once those have left, waves 4-7 issue their weight loads of the
-// phase (`mid`) while waves 0-3 wait for the vector, compute the scale and
-// the digit planes, and only then issue theirs.  Returns the scale (in every
-// thread).
+// Digit planes of a vector other blocks (or the attention launch before) wrote
+// (K a multiple of 128, at most kRowT * 4 * kFVecG), by waves 0-3; the scale
+// goes to red[12].  ex: the vector arrives while this runs.  `issued` as in
+// vec_to_lds.
 constexpr int kFVecG = 8;
-template <bool FP8, class Mid>
-__device__ __forceinline__ float vec_digits(const float *x, int K, uint8_t *dig, float *red, QuadSync &q, Mid &&mid)
+template <bool FP8, class Issued>
+__device__ __forceinline__ void vec_digits(const float *x, int K, bool ex, uint8_t *dig, float *red, QuadSync &q,
+                                           const ExWait &wt, Issued &&issued)
 {
     constexpr int ND = FP8 ? kF8Digits : kI8Digits;
     const int tid = threadIdx.x;
     float *stage = dig_stage(dig, ND, K);
-    vec_to_lds(x, stage, K);
-    asm volatile("" ::: "memory");
-    __syncthreads();              // the vector's loads leave before any weight load of the block
-    if (tid >= kRowT) {
-        mid();
-    } else {
-        wait_vmcnt<0>();
-        quad_sync(q);
-        float m = 0.0f;
+    vec_to_lds(x, stage, K, ex, wt, issued);
+    float m = 0.0f;
+#pragma unroll 2
+    for (int i4 = tid; 4 * i4 < K; i4 += kRowT)
+        m = fmaxf(m, f4_absmax(*(const float4 *)(stage + 4 * i4)));
+    const float sc = digit_scale<FP8>(quad_max(m, red + 8, q));
+#pragma unroll 1
+    for (int i4 = tid; 4 * i4 < K; i4 += kRowT) {
+        const float4 x4 = *(const float4 *)(stage + 4 * i4);
+        const float xe[4] = {x4.x, x4.y, x4.z, x4.w};
+        uint32_t word[ND];
+        digit_words<FP8>(xe, sc, word);
 #pragma unroll
-        for (int g = 0; g < kFVecG; g++) {
-            const int i4 = tid + g * kRowT;
-            if (4 * i4 < K)
-                m = fmaxf(m, f4_absmax(*(const float4 *)(stage + 4 * i4)));
-        }
-        const float sc = digit_scale<FP8>(quad_max(m, red + 8, q));
-#pragma unroll
-        for (int g = 0; g < kFVecG; g++) {
-            const int i4 = tid + g * kRowT;
-            if (4 * i4 < K) {
-                const float4 x4 = *(const float4 *)(stage + 4 * i4);
-                const float xe[4] = {x4.x, x4.y, x4.z, x4.w};
-                uint32_t word[ND];
-                digit_words<FP8>(xe, sc, word);
-#pragma unroll
-                for (int d = 0; d < ND; d++)
-                    *(uint32_t *)(dig + (size_t)d * K + 4 * i4) = word[d];
-            }
-        }
-        if (tid == 0)
-            red[12] = sc;
-        asm volatile("" ::: "memory");
-        mid();
+        for (int d = 0; d < ND; d++)
+            *(uint32_t *)(dig + (size_t)d * K + 4 * i4) = word[d];
     }
-    __syncthreads();
-    return red[12];
+    if (tid == 0)
+        red[12] = sc;
 }
 
-// x + delta (both written by other blocks), RMSNorm with w, into digit
-// planes, with the work split as in vec_digits; block b writes its share of
-// x + delta to x_out.  Threads < kRowT (waves 0-3) hold the row exactly as
-// k_rmsnorm's threads do (same sum of squares, same reduction tree).  EMB:
-// the row is instead the embedding of er's token, formed as k_embed forms it
-// (x and delta unused).
-template <bool FP8, int NV, bool EMB = false, class Mid>
-__device__ __forceinline__ float norm_digits(const float *x, const float *delta, const uint16_t *w, float *x_out,
-                                             int dim, float eps, uint8_t *dig, float *red, int b, int nb,
-                                             QuadSync &q, Mid &&mid, const EmbRow &er = EmbRow{})
+// x + delta, RMSNorm with w, into digit planes, by waves 0-3; the scale goes
+// to red[12].  delta is an exchange buffer, x the layer's input from memory or
+// (null) what the phase before left in hbuf, each thread its own floats.  hbuf
+// takes x + delta; block b writes its share of it to x_out if that is set.
+// The threads hold the row exactly as k_rmsnorm's threads do (same sum of
+// squares, same reduction tree).  EMB: the row is instead the embedding of
+// er's token, formed as k_embed forms it (x and delta unused).
+template <bool FP8, int NV, bool EMB, class Issued>
+__device__ __forceinline__ void norm_digits(const float *x, const float *delta, const uint16_t *w, float *x_out,
+                                            float4 *hbuf, int dim, float eps, uint8_t *dig, float *red, int b, int nb,
+                                            QuadSync &q, const ExWait &wt, const EmbRow &er, Issued &&issued)
 {
     constexpr int ND = FP8 ? kF8Digits : kI8Digits;
     const int tid = threadIdx.x, n4 = dim >> 2;
-    float *sx_ = dig_stage(dig, ND, dim), *sd_ = sx_ + dim;
-    if constexpr (!EMB) {
-        vec_to_lds(x, sx_, dim);
-        vec_to_lds(delta, sd_, dim);
-    }
-    asm volatile("" ::: "memory");
-    __syncthreads();              // the vectors' loads leave before any weight load of the block
-    if (tid >= kRowT) {
-        mid();
+    float *sd_ = dig_stage(dig, ND, dim);
+    float4 v[NV], h[NV];
+    uint2 wv[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++)
+        wv[j] = ((const uint2 *)w)[min(tid + kRowT * j, n4 - 1)];
+    if constexpr (EMB) {
+        issued();
+        const int tok = *er.tok;
+        const float es = er.scale[tok];
+        const uint8_t *row = er.emb + (size_t)tok * dim;
+        auto dq = [](uint32_t c) { return FP8 ? fp8_to_f32((uint8_t)c) : (float)(int8_t)(uint8_t)c; };
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            const int i = min(tid + kRowT * j, n4 - 1);
+            const uint32_t c4 = *(const uint32_t *)(row + 4 * i);
+            v[j] = make_float4(dq(c4 & 0xFFu) * es, dq((c4 >> 8) & 0xFFu) * es, dq((c4 >> 16) & 0xFFu) * es,
+                               dq(c4 >> 24) * es);
+        }
     } else {
-        float4 v[NV], h[NV];
-        uint2 wv[NV];
-        if constexpr (EMB) {
-            const int tok = *er.tok;
-            const float es = er.scale[tok];
-            const uint8_t *row = er.emb + (size_t)tok * dim;
-            auto dq = [](uint32_t c) { return FP8 ? fp8_to_f32((uint8_t)c) : (float)(int8_t)(uint8_t)c; };
+        if (x) {
 #pragma unroll
-            for (int j = 0; j < NV; j++) {
-                const int i = min(tid + kRowT * j, n4 - 1);
-                const uint32_t c4 = *(const uint32_t *)(row + 4 * i);
-                v[j] = make_float4(dq(c4 & 0xFFu) * es, dq((c4 >> 8) & 0xFFu) * es, dq((c4 >> 16) & 0xFFu) * es,
-                                   dq(c4 >> 24) * es);
-                wv[j] = ((const uint2 *)w)[i];
-            }
+            for (int j = 0; j < NV; j++)
+                v[j] = ((const float4 *)x)[min(tid + kRowT * j, n4 - 1)];
         } else {
-            wait_vmcnt<0>();
-            quad_sync(q);
 #pragma unroll
-            for (int j = 0; j < NV; j++) {
-                const int i = min(tid + kRowT * j, n4 - 1);
-                const float4 xv = *(const float4 *)(sx_ + 4 * i), dv = *(const float4 *)(sd_ + 4 * i);
-                v[j] = make_float4(xv.x + dv.x, xv.y + dv.y, xv.z + dv.z, xv.w + dv.w);
-                wv[j] = ((const uint2 *)w)[i];
-            }
+            for (int j = 0; j < NV; j++)
+                v[j] = hbuf[tid + kRowT * j];
         }
-        float ss = 0.0f;
+        vec_to_lds(delta, sd_, dim, true, wt, issued);
 #pragma unroll
         for (int j = 0; j < NV; j++) {
-            const int i = tid + kRowT * j;
-            if (i < n4 && i % nb == b) {
-                float *o = x_out + 4 * i;
-                st_dev(o, v[j].x);
-                st_dev(o + 1, v[j].y);
-                st_dev(o + 2, v[j].z);
-                st_dev(o + 3, v[j].w);
-            }
-            if (i >= n4)
-                v[j] = f4_zero();
-            ss = __fmaf_rn(v[j].x, v[j].x, ss);
-            ss = __fmaf_rn(v[j].y, v[j].y, ss);
-            ss = __fmaf_rn(v[j].z, v[j].z, ss);
-            ss = __fmaf_rn(v[j].w, v[j].w, ss);
+            const float4 dv = *(const float4 *)(sd_ + 4 * min(tid + kRowT * j, n4 - 1));
+            v[j] = make_float4(v[j].x + dv.x, v[j].y + dv.y, v[j].z + dv.z, v[j].w + dv.w);
+            hbuf[tid + kRowT * j] = v[j];
         }
-        ss = wave_sum_dpp(ss);
-        if ((tid & 63) == 0)
-            red[tid >> 6] = ss;
-        quad_sync(q);
-        const float tot = (red[0] + red[1]) + (red[2] + red[3]);
-        const float inv = __fdiv_rn(1.0f, sqrtf(__fdiv_rn(tot, (float)dim) + eps));
-        float m = 0.0f;
-#pragma unroll
-        for (int j = 0; j < NV; j++) {
-            const uint2 wj = wv[j];
-            h[j] = make_float4((v[j].x * inv) * bf16_to_f32((uint16_t)(wj.x & 0xFFFF)),
-                               (v[j].y * inv) * bf16_to_f32((uint16_t)(wj.x >> 16)),
-                               (v[j].z * inv) * bf16_to_f32((uint16_t)(wj.y & 0xFFFF)),
-                               (v[j].w * inv) * bf16_to_f32((uint16_t)(wj.y >> 16)));
-            if (tid + kRowT * j >= n4)
-                h[j] = f4_zero();
-            m = fmaxf(m, f4_absmax(h[j]));
-        }
-        const float sc = digit_scale<FP8>(quad_max(m, red + 8, q));
-#pragma unroll
-        for (int j = 0; j < NV; j++) {
-            const int i = tid + kRowT * j;
-            if (i < n4) {
-                const float xe[4] = {h[j].x, h[j].y, h[j].z, h[j].w};
-                uint32_t word[ND];
-                digit_words<FP8>(xe, sc, word);
-#pragma unroll
-                for (int d = 0; d < ND; d++)
-                    *(uint32_t *)(dig + (size_t)d * dim + 4 * i) = word[d];
-            }
-        }
-        if (tid == 0)
-            red[12] = sc;
-        asm volatile("" ::: "memory");
-        mid();
     }
-    __syncthreads();
-    return red[12];
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = tid + kRowT * j;
+        if (x_out && i < n4 && i % nb == b)
+            ((float4 *)x_out)[i] = v[j];
+        if (i >= n4)
+            v[j] = f4_zero();
+        ss = __fmaf_rn(v[j].x, v[j].x, ss);
+        ss = __fmaf_rn(v[j].y, v[j].y, ss);
+        ss = __fmaf_rn(v[j].z, v[j].z, ss);
+        ss = __fmaf_rn(v[j].w, v[j].w, ss);
+    }
+    ss = wave_sum_dpp(ss);
+    if ((tid & 63) == 0)
+        red[tid >> 6] = ss;
+    quad_sync(q);
+    const float tot = (red[0] + red[1]) + (red[2] + red[3]);
+    const float inv = __fdiv_rn(1.0f, sqrtf(__fdiv_rn(tot, (float)dim) + eps));
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const uint2 wj = wv[j];
+        h[j] = make_float4((v[j].x * inv) * bf16_to_f32((uint16_t)(wj.x & 0xFFFF)),
+                           (v[j].y * inv) * bf16_to_f32((uint16_t)(wj.x >> 16)),
+                           (v[j].z * inv) * bf16_to_f32((uint16_t)(wj.y & 0xFFFF)),
+                           (v[j].w * inv) * bf16_to_f32((uint16_t)(wj.y >> 16)));
+        if (tid + kRowT * j >= n4)
+            h[j] = f4_zero();
+        m = fmaxf(m, f4_absmax(h[j]));
+    }
+    const float sc = digit_scale<FP8>(quad_max(m, red + 8, q));
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = tid + kRowT * j;
+        if (i < n4) {
+            const float xe[4] = {h[j].x, h[j].y, h[j].z, h[j].w};
+            uint32_t word[ND];
+            digit_words<FP8>(xe, sc, word);
+#pragma unroll
+            for (int d = 0; d < ND; d++)
+                *(uint32_t *)(dig + (size_t)d * dim + 4 * i) = word[d];
+        }
+    }
+    if (tid == 0)
+        red[12] = sc;
 }
 
 // The next layer's dense attention for KV head kvh, after this block's K/V
@@ -1058,62 +1039,55 @@ __global__ __launch_bounds__(kFT, 1) void k_fused_layer(const FusedArgs A)
     __shared__ float ybuf[kFMaxTiles * 16];
     __shared__ float red[16];
     __shared__ int qcnt;
+    __shared__ float4 hbuf[START ? 1 : NV * kRowT];   // the layer's h, each thread of waves 0-3 its own floats
     const int b = blockIdx.x, nb = gridDim.x;
     if (threadIdx.x == 0)
         qcnt = 0;
     __syncthreads();
-    QuadSync quad{&qcnt, 0, A.err};
-    GridBar gb{A.flags, __hip_atomic_load(A.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * kFBars, nb, A.err,
-               A.spin_max, A.bias};
+    const ExWait wt = A.wait;
+    QuadSync quad{&qcnt, 0, wt.err};
     v8i fr[kFMaxU];
 #pragma unroll
     for (int u = 0; u < kFMaxU; u++)
         fr[u] = v8i{0, 0, 0, 0, 0, 0, 0, 0};
-    // A phase's input vector is loaded first (waves 0-3); then waves 4-7
-    // issue their weight loads of the phase while waves 0-3 compute the
-    // digit planes, and waves 0-3 issue theirs after (a vector load queued
-    // behind the phase's weight stream would hold up the digits).
-    auto wload = [&](const FPhase &ph) {
-        const FPhase *pp = &ph;
-        return [pp, b, nb, &fr] { ph_prefetch(*pp, b, nb, fr, 0, kFW); };
+    // empties the exchange buffers a later launch will use (waves 4-7)
+    auto clear = [&] {
+        if (threadIdx.x >= kRowT)
+            for (int c = 0; c < 2; c++)
+                for (int i = (threadIdx.x - kRowT) * nb + b; i < A.nclr[c]; i += kRowT * nb)
+                    st_dev(A.clr[c] + i, __uint_as_float(kFEmpty));
     };
-    FOut oo;
-    float sx;
-    if constexpr (!START) {
-        // o projection of the attention output
-        oo = ph_out(A.o, b, nb);
-        sx = vec_digits<FP8>(A.att, A.qd, dig, red, quad, wload(A.o));
-        ph_compute<FP8>(A.o, b, nb, fr, dig, A.qd, sx, part, ybuf, oo);
-        grid_barrier(gb, 1, [] {});
-        // h = x + o, RMSNorm, gate/up, SiLU * up
-        oo = ph_out(A.gu, b, nb);
-        sx = norm_digits<FP8, NV>(A.X, A.XB, A.ffn_norm, A.Hb, A.dim, A.eps, dig, red, b, nb, quad, wload(A.gu));
-        ph_compute<FP8>(A.gu, b, nb, fr, dig, A.dim, sx, part, ybuf, oo);
-        grid_barrier(gb, 2, [] {});
-        // down projection
-        oo = ph_out(A.down, b, nb);
-        sx = vec_digits<FP8>(A.H2, A.hidden, dig, red, quad, wload(A.down));
-        ph_compute<FP8>(A.down, b, nb, fr, dig, A.hidden, sx, part, ybuf, oo);
-        if (A.qkv.nseg == 0) {
-            // last layer: h and the down output stay for the final norm
-            if (b == 0 && threadIdx.x == 0)
-                __hip_atomic_store(A.gen, gb.base / kFBars + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return;
+    // One copy of the phases' code (unrolled, the kernel is 98 KB of
+    // instructions that run once a launch, more than the instruction cache,
+    // and each miss is a trip past an L2 that the weights have swept).
+#pragma unroll 1
+    for (int p = START ? 3 : 0;; p++) {
+        const FPhase &ph = A.ph[p];
+        const FOut oo = ph_out(ph, b, nb);
+        if (threadIdx.x >= kRowT) {
+            lds_barrier();
+        } else if (START || (p & 1)) {
+            // phase 1: h = x + o, RMSNorm, gate/up, SiLU * up; phase 3: the next
+            // layer's x = h + down (the step's first launch: the token's
+            // embedding), RMSNorm, q/k/v
+            norm_digits<FP8, NV, START>(p == 1 ? A.X : nullptr, p == 1 ? A.ex_o : A.ex_dn,
+                                        p == 1 ? A.ffn_norm : A.attn_norm,
+                                        p == 3 || A.last == 2 ? A.Xout : nullptr, hbuf, A.dim, A.eps, dig, red, b, nb,
+                                        quad, wt, A.er, [] { lds_barrier(); });
+        } else {
+            // phase 0: the o projection of the attention output; phase 2: down
+            vec_digits<FP8>(p == 0 ? A.att : A.ex_h2, ph.K, p != 0, dig, red, quad, wt, [] { lds_barrier(); });
         }
-        grid_barrier(gb, 3, [] {});
+        asm volatile("" ::: "memory");
+        ph_prefetch(ph, b, nb, fr, 0, kFW);
+        lds_barrier();
+        ph_compute<FP8>(ph, b, nb, fr, dig, ph.K, red[12], part, ybuf, oo);
+        if (p == A.last)
+            break;
     }
-    // next layer: x = h + down (the step's first launch: x = the token's
-    // embedding), RMSNorm, q/k/v
-    oo = ph_out(A.qkv, b, nb);
-    if constexpr (START)
-        sx = norm_digits<FP8, NV, true>(nullptr, nullptr, A.attn_norm, A.X, A.dim, A.eps, dig, red, b, nb, quad,
-                                        wload(A.qkv), A.er);
-    else
-        sx = norm_digits<FP8, NV>(A.Hb, A.XB, A.attn_norm, A.X, A.dim, A.eps, dig, red, b, nb, quad, wload(A.qkv));
-    ph_compute<FP8>(A.qkv, b, nb, fr, dig, A.dim, sx, part, ybuf, oo);
-    grid_barrier(gb, 4, [] {});
-    if (b == 0 && threadIdx.x == 0)
-        __hip_atomic_store(A.gen, gb.base / kFBars + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    clear();
+    if (!START && A.last == 2)
+        return;   // the last layer: h and the down output stay for the final norm
     if (b >= A.KV) {
         if (A.pf_route && b < A.KV + 8 && threadIdx.x < kWave) {
             // Blocks KV .. KV + 7 (one per XCD; they have no tail): the next
@@ -1137,12 +1111,18 @@ __global__ __launch_bounds__(kFT, 1) void k_fused_layer(const FusedArgs A)
     // RoPE of the q heads of KV head b and of k head b, K/V append and seal
     const int hd = A.P.head_dim, half = hd / 2, G = A.H / A.KV, tid = threadIdx.x;
     float *qs = (float *)dig, *ks = qs + G * hd, *vs = ks + hd, *cs = vs + hd;
-    float *qrow = A.q + (size_t)b * G * hd, *krow = A.k + (size_t)b * hd;
-    for (int i = tid; i < G * hd; i += kFT)
-        qs[i] = ld_dev(qrow + i);
-    for (int i = tid; i < hd; i += kFT) {
-        ks[i] = ld_dev(krow + i);
-        vs[i] = ld_dev(A.v + (size_t)b * hd + i);
+    float *qrow = A.q + (size_t)b * G * hd, *krow = A.k + (size_t)b * hd, *vrow = A.v + (size_t)b * hd;
+    for (int i = tid; i < (G + 2) * hd; i += kFT) {
+        const float *src = i < G * hd         ? A.ex_q + (size_t)b * G * hd + i
+                           : i < (G + 1) * hd ? A.ex_k + (size_t)b * hd + (i - G * hd)
+                                              : A.ex_v + (size_t)b * hd + (i - (G + 1) * hd);
+        float y = ld_dev(src);
+        for (unsigned spins = 1; __float_as_uint(y) == kFEmpty || wt.never; spins++) {
+            if (ex_give_up(wt, spins))
+                break;
+            y = ld_dev(src);
+        }
+        qs[i] = y;   // q, k and v rows lie behind each other
     }
     __syncthreads();
     const int pos = *A.pos_p;
@@ -1160,8 +1140,10 @@ __global__ __launch_bounds__(kFT, 1) void k_fused_layer(const FusedArgs A)
     // the rotated rows for the attention launch that follows (and captures)
     for (int i = tid; i < G * hd; i += kFT)
         qrow[i] = qs[i];
-    for (int i = tid; i < hd; i += kFT)
+    for (int i = tid; i < hd; i += kFT) {
         krow[i] = ks[i];
+        vrow[i] = vs[i];
+    }
     if (A.app->n > 0)
         append_seal_tail<BF16KV>(A.P, *A.app, 0, b, ks, vs, cs);
     if (A.att_out) {
@@ -1225,12 +1207,13 @@ struct be42_decoder {
     } key[2];
     hipGraphExec_t exec[2] = {nullptr, nullptr};
     bool use_graph = true;
-    // the fused layer of one-sequence steps: grid = the CU count; barrier
-    // flags [(nb + 1) * 32], launch counter, error flag (device, zeroed at create)
+    // the fused layer of one-sequence steps: grid = the CU count; exchange
+    // buffers (FusedEx) and the second residual buffer
     bool fused = false;
-    bool fail_barriers = false;   // test: every grid-barrier wait gives up
+    bool fail_barriers = false;   // test: every wait of the fused launches gives up
     int fnb = 0;
-    unsigned *fflags = nullptr;
+    float *fex = nullptr;
+    bool fex_dirty = false;       // a step ended half-way through its launches: empty fex before the next
     // a fused launch's error flag seen set: the decoder's state is invalid and
     // every later step or prefill is refused (the device flag stays set)
     int fault = 0;
@@ -1245,6 +1228,22 @@ struct be42_decoder {
     // the chunk's page selections [kPrefillChunk][psel_stride] and counts
     int *psel = nullptr, *pnsel = nullptr;
     int psel_stride = 0;
+};
+
+// The exchange buffers of the fused launches in be42_decoder::fex, two sets of
+// each since a launch empties what the launch before it used: o, down and
+// gate/up outputs (layer l: set l % 2), then q, k, v (layer l's rows, written
+// by the launch before: set l % 2); after them the residual stream of the odd
+// layers.
+struct FusedEx {
+    size_t ffn, qkv;   // floats of a set
+    explicit FusedEx(const be42_decoder_config &c)
+        : ffn((size_t)2 * c.dim + c.hidden_dim), qkv((size_t)(c.n_heads + 2 * c.n_kv_heads) * c.head_dim)
+    {
+    }
+    size_t ffn_at(int l) const { return (size_t)(l & 1) * ffn; }
+    size_t qkv_at(int l) const { return 2 * ffn + (size_t)(l & 1) * qkv; }
+    size_t x_at() const { return 2 * (ffn + qkv); }
 };
 
 // Whether the fused layer kernel serves this shape at batch 1 (sets d->fnb).
@@ -1396,10 +1395,10 @@ extern "C" int be42_decoder_create(be42_decoder **out, const be42_decoder_config
     if (e == hipSuccess && fused_layer_fits(c, d)) {
         const char *fz = getenv("BE42_DECODE_FUSED");
         if (!(fz && fz[0] == '0')) {
-            const size_t fbytes = ((size_t)d->fnb + 1) * 128 + 256;
-            e = hipMalloc((void **)&d->fflags, fbytes);
+            const FusedEx fx(d->c);
+            e = hipMalloc((void **)&d->fex, (fx.x_at() + d->c.dim) * 4);
             if (e == hipSuccess)
-                e = hipMemset(d->fflags, 0, fbytes);
+                e = hipMemset(d->fex, 0xFF, fx.x_at() * 4);   // kFEmpty
             d->fused = e == hipSuccess;
             const char *fb = getenv("BE42_DECODE_FAIL_BARRIERS");
             d->fail_barriers = fb && fb[0] == '1';
@@ -1444,7 +1443,7 @@ extern "C" void be42_decoder_destroy(be42_decoder *d)
     if (d->pmeta_host)
         (void)hipHostFree(d->pmeta_host);
     void *ptrs[] = {d->cos_t, d->sin_t, d->x, d->xb, d->xn, d->q, d->k, d->v, d->att, d->hb, d->hb2, d->logits, d->sel,
-                    d->nsel, d->slots, d->next, d->cand, d->ncand, d->xdig, d->attn_ws, d->arg_parts, d->arg_cnt, d->fflags,
+                    d->nsel, d->slots, d->next, d->cand, d->ncand, d->xdig, d->attn_ws, d->arg_parts, d->arg_cnt, d->fex,
                     d->px, d->pxn, d->pq, d->pk, d->pv, d->patt, d->pxb, d->phb, d->phb2, d->pdig, d->pmeta,
                     d->psel, d->pnsel};
     for (void *p : ptrs)
@@ -1530,40 +1529,56 @@ static int launch_fused_layer(be42_decoder *d, int l, const AppendStepArgs *app,
     const be42_decoder_layer &L = d->w.layers[start ? 0 : l];
     const int dim = c.dim, hidden = c.hidden_dim, qd = c.n_heads * c.head_dim, kd = c.n_kv_heads * c.head_dim;
     FusedArgs A{};
-    A.o = one_phase(L.wo, L.so, d->xb, dim, qd);
-    A.gu = one_phase(L.w1, L.s1, d->hb, hidden, dim);
-    A.gu.w[1] = (const uint8_t *)L.w3;
-    A.gu.sw[1] = L.s3;
-    A.gu.n[1] = hidden;
-    A.gu.nseg = 2;
-    A.gu.silu = 1;
-    A.down = one_phase(L.w2, L.s2, d->xb, dim, hidden);
-    if (start || l + 1 < c.n_layers) {
-        const be42_decoder_layer &N = d->w.layers[start ? 0 : l + 1];
-        A.qkv = one_phase(N.wq, N.sq, d->q, qd, dim);
-        A.qkv.w[1] = (const uint8_t *)N.wk;
-        A.qkv.w[2] = (const uint8_t *)N.wv;
-        A.qkv.sw[1] = N.sk;
-        A.qkv.sw[2] = N.sv;
-        A.qkv.y[1] = d->k;
-        A.qkv.y[2] = d->v;
-        A.qkv.n[1] = A.qkv.n[2] = kd;
-        A.qkv.nseg = 3;
-        A.qkv.tend[0] = qd / 16;
-        A.qkv.tend[1] = qd / 16 + kd / 16;
-        A.qkv.tend[2] = qd / 16 + 2 * (kd / 16);
-        A.qkv.units = A.qkv.tend[2];
+    const FusedEx fx(c);
+    const bool last = !start && l + 1 == c.n_layers;
+    const int next = start ? 0 : l + 1;   // the layer whose q, k, v this launch computes
+    float *ex = d->fex + (start ? 0 : fx.ffn_at(l)), *exq = d->fex + fx.qkv_at(next);
+    float *x[2] = {d->x, d->fex + fx.x_at()};
+    A.ph[0] = one_phase(L.wo, L.so, ex, dim, qd);
+    A.ph[1] = one_phase(L.w1, L.s1, ex + 2 * dim, hidden, dim);
+    A.ph[1].w[1] = (const uint8_t *)L.w3;
+    A.ph[1].sw[1] = L.s3;
+    A.ph[1].n[1] = hidden;
+    A.ph[1].nseg = 2;
+    A.ph[1].silu = 1;
+    A.ph[2] = one_phase(L.w2, L.s2, last ? d->xb : ex + dim, dim, hidden);
+    if (!last) {
+        const be42_decoder_layer &N = d->w.layers[next];
+        A.ph[3] = one_phase(N.wq, N.sq, exq, qd, dim);
+        A.ph[3].w[1] = (const uint8_t *)N.wk;
+        A.ph[3].w[2] = (const uint8_t *)N.wv;
+        A.ph[3].sw[1] = N.sk;
+        A.ph[3].sw[2] = N.sv;
+        A.ph[3].y[1] = exq + qd;
+        A.ph[3].y[2] = exq + qd + kd;
+        A.ph[3].n[1] = A.ph[3].n[2] = kd;
+        A.ph[3].nseg = 3;
+        A.ph[3].tend[0] = qd / 16;
+        A.ph[3].tend[1] = qd / 16 + kd / 16;
+        A.ph[3].tend[2] = qd / 16 + 2 * (kd / 16);
+        A.ph[3].units = A.ph[3].tend[2];
         A.attn_norm = N.attn_norm;
-        A.app = app + (start ? 0 : l + 1);
+        A.app = app + next;
     } else {
-        A.qkv.nseg = 0;
+        A.ph[3].nseg = 0;
         A.app = app + l;
     }
+    A.last = last ? 2 : 3;
     A.att = d->att;
-    A.X = d->x;
-    A.Hb = d->xn;
-    A.XB = d->xb;
-    A.H2 = d->hb;
+    A.ex_o = ex;
+    A.ex_dn = ex + dim;
+    A.ex_h2 = ex + 2 * dim;
+    A.ex_q = exq;
+    A.ex_k = exq + qd;
+    A.ex_v = exq + qd + kd;
+    // what the launch before used; the step's first launch empties the last
+    // layer's ffn set (which used no q, k, v)
+    A.clr[0] = d->fex + fx.ffn_at(start ? c.n_layers - 1 : l + 1);
+    A.nclr[0] = (int)fx.ffn;
+    A.clr[1] = d->fex + fx.qkv_at(l);
+    A.nclr[1] = start ? 0 : (int)fx.qkv;
+    A.X = start ? nullptr : x[l & 1];
+    A.Xout = last ? d->xn : x[next & 1];
     A.q = d->q;
     A.k = d->k;
     A.v = d->v;
@@ -1580,15 +1595,11 @@ static int launch_fused_layer(be42_decoder *d, int l, const AppendStepArgs *app,
     A.H = c.n_heads;
     A.KV = c.n_kv_heads;
     A.eps = c.norm_eps;
-    A.flags = d->fflags;
-    A.gen = d->fflags + ((size_t)d->fnb + 1) * 32;
-    A.err = d->next + kMaxBatch;
-    A.spin_max = d->fail_barriers ? 64u : kFSpinMax;
-    A.bias = d->fail_barriers ? 1u << 24 : 0u;
-    A.att_out = start || l + 1 < c.n_layers ? att_out : nullptr;
+    A.wait = ExWait{d->next + kMaxBatch, d->fail_barriers ? 64u : kFSpinMax, d->fail_barriers};
+    A.att_out = last ? nullptr : att_out;
     A.att_scale = att_scale;
     A.er = EmbRow{(const uint8_t *)d->w.emb, d->w.emb_s, start_tok};
-    A.pf_route = pf_route && (start || l + 1 < c.n_layers);
+    A.pf_route = pf_route && !last;
     const int nv = (dim + kChunk - 1) / kChunk;
     const bool fp8 = c.wkind != 0, bf16 = c.kv_kind == BE42_KV_BF16;
     auto go = [&](auto f8, auto kb, auto nvc) {
@@ -1799,7 +1810,7 @@ static int fault_check(be42_decoder *d, bool wait, const char *what)
         }
     }
     BE42_CHECK(d->fault == 0,
-               "%s: a bounded wait gave up in an earlier step (code %d: 1-2 a grid barrier of the fused layer, 3 its "
+               "%s: a bounded wait gave up in an earlier step (code %d: 1 a grid barrier of the fused layer, 3 its "
                "wave sync, 4 the split attention's); the decoder's results and cache are invalid (destroy it)",
                what, d->fault);
     return BE42_OK;
@@ -1883,9 +1894,15 @@ static int launch_step(be42_decoder *d, int B, int pos, bool host_tokens, float 
     hipStream_t st = d->gstream;
     BE42_HIP(hipEventRecord(d->ev_in, caller));
     BE42_HIP(hipStreamWaitEvent(st, d->ev_in, 0));
+    if (d->fex_dirty) {
+        BE42_HIP(hipMemsetAsync(d->fex, 0xFF, FusedEx(c).x_at() * 4, st));
+        d->fex_dirty = false;
+    }
     if (!d->use_graph) {
         *queued = true;   // launched one by one: a failure can come after some of them
+        d->fex_dirty = d->fused;
         DEC_TRY(enqueue_step(d, B, key.sparse, key.dev_tokens, logits_out, par, st));
+        d->fex_dirty = false;
     } else {
         if (!d->exec[par] || !(d->key[par] == key)) {
             if (d->exec[par]) {

@@ -252,8 +252,7 @@ def test_graph_replay_matches_eager(be, orc, monkeypatch):
 @pytest.mark.parametrize("kind,kv_kind", [("int8", OR_KV_INT8), ("int8", OR_KV_BF16), ("fp8", OR_KV_BF16)])
 def test_fused_layer_matches_separate_launches(be, orc, monkeypatch, kind, kv_kind):
     """The one-sequence fused layer launch (o, norm, gate/up + SiLU, down and
-    the next layer's norm, q/k/v, RoPE and append in one launch with grid
-    barriers) against the same steps with separate launches
+    the next layer's norm, q/k/v, RoPE and append in one launch) against the same steps with separate launches
     (BE42_DECODE_FUSED=0): 4 layers, d 512, sparse_k 8 so that every position
     past 128 routes; 200 prompt tokens, then 20 greedy steps.  INT8 weights:
     the logits of every step bit-identical (same arithmetic, exact digit
@@ -320,6 +319,64 @@ def test_fused_layer_group3_matches_separate_launches(be, orc, monkeypatch, kv_k
     monkeypatch.delenv("BE42_DECODE_FUSED")
     l1 = run()
     np.testing.assert_array_equal(l0, l1)
+
+
+@pytest.mark.parametrize("n_layers,dim,hidden", [(1, 512, 1408), (2, 1152, 128), (3, 512, 2048), (3, 640, 1408)])
+def test_fused_layer_exchange(be, orc, monkeypatch, n_layers, dim, hidden):
+    """The fused launches hand vectors on through buffers that the next launch
+    empties, two sets in turn: odd and even layer counts, rows that are no
+    multiple of a wave's 1 KB chunk (1152 and 640 floats) and phases with
+    fewer tiles than blocks, ten steps, with steps of the separate launches
+    (two sequences) between them: bit-identical to BE42_DECODE_FUSED=0."""
+    rng = np.random.default_rng(n_layers * dim)
+    w = make_model(rng, n_layers, dim, 8, 4, 64, hidden, 512, "int8")
+    _, gc = configs(n_layers, dim, 8, 4, 64, hidden, 512, 64, 2, "int8", OR_KV_INT8, 8, 64)
+    _, hpT = orc.lsh_init(64, 42)
+    wd = to_device(w)
+
+    def run():
+        dec = be42.Decoder(be, gc, wd, hpT)
+        lg, out = torch.empty((2, 512), device="cuda"), []
+        for pos in range(10):
+            toks = [3 + pos, 7 * pos] if pos in (4, 5) else [3 + pos]
+            dec.step(toks, pos if len(toks) == 1 else pos - 4, logits=lg)
+            out.append(lg[:len(toks)].cpu().numpy().copy())
+        dec.status()
+        dec.close()
+        return np.concatenate(out)
+
+    monkeypatch.setenv("BE42_DECODE_FUSED", "0")
+    want = run()
+    monkeypatch.delenv("BE42_DECODE_FUSED")
+    np.testing.assert_array_equal(run(), want)
+
+
+@pytest.mark.parametrize("name", ["so", "s1", "s2", "sv"])
+def test_fused_layer_passes_nan_on(be, orc, monkeypatch, name):
+    """A NaN whose bits are all ones (what an empty exchange word holds) is a
+    value like any other: with a row scale of that NaN no wait gives up and
+    two steps equal those of the separate launches."""
+    rng = np.random.default_rng(9)
+    w = make_model(rng, 2, 512, 8, 8, 64, 1408, 512, "int8")
+    _, gc = configs(2, 512, 8, 8, 64, 1408, 512, 64, 1, "int8", OR_KV_BF16, 8, 64)
+    _, hpT = orc.lsh_init(64, 42)
+    wd = to_device(w)
+    wd["layers"][1 if name == "sv" else 0][name].view(torch.int32)[5] = -1
+
+    def run():
+        dec = be42.Decoder(be, gc, wd, hpT)
+        lg, out = torch.empty((1, 512), device="cuda"), []
+        for pos in range(2):
+            dec.step([1 + pos], pos, logits=lg)
+            out.append(lg.cpu().numpy().copy())
+        dec.status()
+        dec.close()
+        return np.concatenate(out)
+
+    monkeypatch.setenv("BE42_DECODE_FUSED", "0")
+    want = run()
+    monkeypatch.delenv("BE42_DECODE_FUSED")
+    np.testing.assert_array_equal(run(), want)
 
 
 def test_barrier_timeout_is_reported(be, orc, monkeypatch):
