@@ -437,8 +437,8 @@ __global__ __launch_bounds__(256) void k_rope_rows(float *__restrict__ q, float 
 // digit planes; waves 4-7 issue their weight loads of the phase as soon as the
 // first of these reads have left, so that weights stream while the block waits.
 // Norm weights and row scales are loaded before the vector.  3B layer (FP8, 100.8
-// MB) 48.4 -> 41.2 us, its step 2250 -> 2046; 4-layer INT8 step of 512 / 1408
-// floats 222 -> 191.
+// MB) 48.4 -> 40 us, its step 2250 -> 2013; 4-layer INT8 step of 512 / 1408 floats
+// 222 -> 187.
 //
 // Coherence: exchanged words go through device-scope (agent) stores and loads,
 // which act at the device's coherence point.  Each word stands for itself, so
@@ -826,7 +826,8 @@ __device__ __forceinline__ float *dig_stage(uint8_t *dig, int nd, int K)
 // Waves 0-3 of a block wait for each other through an LDS counter (waves
 // 4-7 take no part: they may be stalled issuing weight loads, and a block
 // barrier would hold waves 0-3 behind them).  Every call adds 4 to the
-// target; the wait is bounded like the exchange's.
+// target; the wait is bounded like the exchange's.  The four waves are at most a
+// few hundred cycles apart: they poll without sleeping (3B step 2024 -> 2015 us).
 struct QuadSync {
     int *cnt;     // LDS, 0 at kernel start
     int target;
@@ -840,8 +841,7 @@ __device__ __forceinline__ void quad_sync(QuadSync &q)
         __hip_atomic_fetch_add(q.cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     unsigned spins = 0;
     while (__hip_atomic_load(q.cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < q.target) {
-        __builtin_amdgcn_s_sleep(1);
-        if (++spins > kFSpinMax * 16) {
+        if (++spins > kFSpinMax * 64) {
             if ((threadIdx.x & 63) == 0)
                 atomicExch(q.err, 3);
             break;
@@ -850,10 +850,23 @@ __device__ __forceinline__ void quad_sync(QuadSync &q)
     asm volatile("" ::: "memory");
 }
 
+// wave_max with DPP lane moves instead of six trips through the LDS crossbar;
+// lanes without a source keep their own value (3B step 2024 -> 2007 us)
+__device__ __forceinline__ float wave_max_dpp(float v)
+{
+    v = fmaxf(v, dpp_mov<0x111>(v, v));
+    v = fmaxf(v, dpp_mov<0x112>(v, v));
+    v = fmaxf(v, dpp_mov<0x114>(v, v));
+    v = fmaxf(v, dpp_mov<0x118>(v, v));
+    v = fmaxf(v, dpp_mov<0x142, 0xA>(v, v));
+    v = fmaxf(v, dpp_mov<0x143, 0xC>(v, v));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
 // max over waves 0-3 of a per-lane value (red: 4 floats of LDS)
 __device__ __forceinline__ float quad_max(float v, float *red, QuadSync &q)
 {
-    v = wave_max(v);
+    v = wave_max_dpp(v);
     if ((threadIdx.x & 63) == 0)
         red[threadIdx.x >> 6] = v;
     quad_sync(q);
