@@ -434,10 +434,10 @@ __global__ __launch_bounds__(256) void k_rope_rows(float *__restrict__ q, float 
 // buffer until no word is empty: one trip out and one in, with no wait for the
 // stores, no arrival flags and no release flag (which took 2.2 - 2.6 us a phase,
 // and 1.8 for the vector after it).  Waves 0-3 read the vector and compute the
-// digit planes; waves 4-7 issue their weight loads of the phase as soon as the
-// first of these reads have left, so that weights stream while the block waits.
+// digit planes; waves 4-7 issue their weight loads of the phase kFWeightWait after
+// the first of these reads have left, so that weights stream meanwhile.
 // Norm weights and row scales are loaded before the vector.  3B layer (FP8, 100.8
-// MB) 48.4 -> 40 us, its step 2250 -> 2013; 4-layer INT8 step of 512 / 1408 floats
+// MB) 48.4 -> 38 us, its step 2243 -> 1959; 4-layer INT8 step of 512 / 1408 floats
 // 222 -> 187.
 //
 // Coherence: exchanged words go through device-scope (agent) stores and loads,
@@ -457,6 +457,7 @@ constexpr int kFW = kFT / kWave;          // waves per block
 constexpr int kFMaxU = 12;                // MFMA steps (128 k-bytes) one wave holds in registers
 constexpr int kFMaxTiles = 8;             // 16-row tiles of one block in one phase
 constexpr int kFDigBytes = 84 * 1024;     // LDS digit planes; also keeps one block per CU
+constexpr int kFWeightWait = 40;          // s_sleep units before waves 4-7 issue weight loads behind an exchange
 constexpr unsigned kFSpinMax = 1u << 16;  // polls (about 1 us each) before a wait gives up
 
 __device__ __forceinline__ float ld_dev(const float *p)
@@ -887,13 +888,25 @@ __device__ __forceinline__ void vec_digits(const float *x, int K, bool ex, uint8
     float *stage = dig_stage(dig, ND, K);
     vec_to_lds(x, stage, K, ex, wt, issued);
     float m = 0.0f;
-#pragma unroll 2
-    for (int i4 = tid; 4 * i4 < K; i4 += kRowT)
-        m = fmaxf(m, f4_absmax(*(const float4 *)(stage + 4 * i4)));
+    // all of a thread's floats in registers: one LDS round trip, not one a
+    // float4 (3B step 1991 -> 1970 us).  Only its own floats: other waves' may
+    // not have arrived.
+    float4 xv[kFVecG];
+#pragma unroll
+    for (int g = 0; g < kFVecG; g++) {
+        const int i4 = tid + g * kRowT;
+        xv[g] = 4 * i4 < K ? *(const float4 *)(stage + 4 * i4) : f4_zero();
+    }
+#pragma unroll
+    for (int g = 0; g < kFVecG; g++)
+        m = fmaxf(m, f4_absmax(xv[g]));
     const float sc = digit_scale<FP8>(quad_max(m, red + 8, q));
-#pragma unroll 1
-    for (int i4 = tid; 4 * i4 < K; i4 += kRowT) {
-        const float4 x4 = *(const float4 *)(stage + 4 * i4);
+#pragma unroll
+    for (int g = 0; g < kFVecG; g++) {
+        const int i4 = tid + g * kRowT;
+        if (4 * i4 >= K)
+            break;
+        const float4 x4 = xv[g];
         const float xe[4] = {x4.x, x4.y, x4.z, x4.w};
         uint32_t word[ND];
         digit_words<FP8>(xe, sc, word);
@@ -1079,6 +1092,12 @@ __global__ __launch_bounds__(kFT, 1) void k_fused_layer(const FusedArgs A)
         const FOut oo = ph_out(ph, b, nb);
         if (threadIdx.x >= kRowT) {
             lds_barrier();
+            // The weight loads fill the CU's memory queue for 1.5 - 3 us, and a
+            // poll behind them waits as long: leave the queue to the polls for
+            // about as long as the vector takes to arrive.  3B step by the sleep
+            // (64 cycles each): 0 1970 us, 12 1946, 24 1947, 40 1924, 80 1992.
+            if (p > 0)
+                __builtin_amdgcn_s_sleep(kFWeightWait);
         } else if (START || (p & 1)) {
             // phase 1: h = x + o, RMSNorm, gate/up, SiLU * up; phase 3: the next
             // layer's x = h + down (the step's first launch: the token's
