@@ -437,7 +437,7 @@ __global__ __launch_bounds__(256) void k_rope_rows(float *__restrict__ q, float 
 // digit planes; waves 4-7 issue their weight loads of the phase kFWeightWait after
 // the first of these reads have left, so that weights stream meanwhile.
 // Norm weights and row scales are loaded before the vector.  3B layer (FP8, 100.8
-// MB) 48.4 -> 38 us, its step 2243 -> 1959; 4-layer INT8 step of 512 / 1408 floats
+// MB) 49.7 -> 40.2 us (trace), its step 2243 -> 1956; 4-layer INT8 step of 512 / 1408 floats
 // 222 -> 187.
 //
 // Coherence: exchanged words go through device-scope (agent) stores and loads,
