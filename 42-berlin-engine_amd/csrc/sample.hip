@@ -231,8 +231,8 @@ struct SelShared {
     unsigned long long hist[BINS];   // bucket sums of a pass
     unsigned long long scan[kSampT / kWave];
     int isum[kSampT / kWave];
-    unsigned long long total, above;
-    int pos, idx;
+    unsigned long long total, above[3];
+    int pos[3], idx;
 };
 using TopPShared = SelShared<kSelBins>;
 
@@ -246,18 +246,35 @@ __device__ __forceinline__ unsigned long long shfl_up_u64(unsigned long long v, 
     return (unsigned long long)hi << 32 | lo;
 }
 
+// inclusive prefix sum over the lanes, as wave_prefix_sum
+template <int CTRL, int ROWMASK = 0xF>
+__device__ __forceinline__ unsigned long long dpp_u64(unsigned long long v)
+{
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, ROWMASK, 0xF, false);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWMASK, 0xF, false);
+    return (unsigned long long)hi << 32 | lo;
+}
+__device__ __forceinline__ unsigned long long wave_prefix_sum_u64(unsigned long long v)
+{
+    v += dpp_u64<0x111>(v);
+    v += dpp_u64<0x112>(v);
+    v += dpp_u64<0x114>(v);
+    v += dpp_u64<0x118>(v);
+    v += dpp_u64<0x142, 0xA>(v);
+    v += dpp_u64<0x143, 0xC>(v);
+    return v;
+}
+
 // Exclusive block scan of one value per thread (thread order of NT); sh: one
-// word per wave.
+// word per wave, free again after the caller's next barrier.  Six passes of a
+// top-p call each wait for one scan and one crossing_bin: through the LDS
+// crossbar, and with four barriers a crossing, a call on a row of 4096 took
+// 42.4 us; with lane moves and one barrier 32.5.
 template <int NT>
 __device__ __forceinline__ unsigned long long block_excl_scan(unsigned long long v, unsigned long long *sh)
 {
     const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
-    unsigned long long incl = v;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        const unsigned long long a = shfl_up_u64(incl, o);
-        incl += lane >= o ? a : 0ull;
-    }
+    const unsigned long long incl = wave_prefix_sum_u64(v);
     if (lane == kWave - 1)
         sh[wave] = incl;
     __syncthreads();
@@ -265,7 +282,6 @@ __device__ __forceinline__ unsigned long long block_excl_scan(unsigned long long
 #pragma unroll
     for (int w = 0; w < NT / kWave; w++)
         before += w < wave ? sh[w] : 0ull;
-    __syncthreads();
     return before + incl - v;
 }
 
@@ -280,6 +296,8 @@ __device__ __forceinline__ BinScan scan_bins(const unsigned long long *hist, int
 {
     BinScan r;
     unsigned long long ts = 0;
+    if (threadIdx.x < 3)
+        S.pos[threadIdx.x] = INT32_MAX;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int d = 4 * (int)threadIdx.x + j;
@@ -292,36 +310,26 @@ __device__ __forceinline__ BinScan scan_bins(const unsigned long long *hist, int
     return r;
 }
 
-// The descending position of the bucket in which base + the running sum first
-// exceeds T (INT32_MAX: none does), *above the sum before that bucket.  Called
-// by the whole block.
+// The descending position of the bucket in which base (at most T) + the
+// running sum first exceeds T (INT32_MAX: none does), *above the sum before
+// that bucket.  Called by the whole block, once per `at` after a scan_bins (the
+// sums do not decrease, so one thread at most has the crossing).
 template <class Sh>
 __device__ __forceinline__ int crossing_bin(const BinScan &r, unsigned long long base, unsigned long long T,
-                                            Sh &S, unsigned long long *above)
+                                            Sh &S, int at, unsigned long long *above)
 {
-    if (threadIdx.x == 0)
-        S.pos = INT32_MAX;
-    __syncthreads();
-    unsigned long long acc = base + r.ex, hit_above = 0;
-    int hit = -1;
+    unsigned long long acc = base + r.ex;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        if (hit < 0 && r.h[j] && acc + r.h[j] > T) {
-            hit = 4 * (int)threadIdx.x + j;
-            hit_above = acc;
+        if (acc <= T && acc + r.h[j] > T) {
+            S.pos[at] = 4 * (int)threadIdx.x + j;
+            S.above[at] = acc;
         }
         acc += r.h[j];
     }
-    if (hit >= 0)
-        atomicMin(&S.pos, hit);
     __syncthreads();
-    const int pos = S.pos;
-    if (hit >= 0 && hit == pos)
-        S.above = hit_above;
-    __syncthreads();
-    *above = S.above;
-    __syncthreads();
-    return pos;
+    *above = S.above[at];
+    return S.pos[at];
 }
 
 // The entry of a list of n probabilities (ld(i): the bits of the i-th, in
@@ -353,7 +361,7 @@ __device__ int weighted_select(Ld &&ld, int n, unsigned long long T, Sh &S, int 
         });
         __syncthreads();
         const BinScan r = scan_bins<NT>(S.hist, nb, S);
-        const int pos = crossing_bin(r, base, T, S, &base);
+        const int pos = crossing_bin(r, base, T, S, 0, &base);
         if (pass == 0)
             *all = S.total;
         if (pos == INT32_MAX)
@@ -473,8 +481,8 @@ __global__ __launch_bounds__(kSampT) void k_top_p(int *__restrict__ out, const f
 // fraction of what a CU can load, and leaves the other CUs idle; here each step
 // of the same computation is a launch of kSlices blocks per row, and after the
 // first pass only the few entries in the buckets of the two crossings are
-// looked at again (k_row_bins, k_row_gather, k_row_pick: 13, 5 and 16 us of the
-// 50 us of 8 rows of 128256).  The results are the same bits: the
+// looked at again (8 rows of 128256: 194 us on one block each, 42 so).  The
+// results are the same bits: the
 // maximum and the 62-bit sums do not depend on the order, and the sum of the
 // exponentials keeps k_probs's (block j sums, row by row of kSampT entries,
 // the 64 columns that wave j of k_probs's block sums).
@@ -618,7 +626,7 @@ __global__ __launch_bounds__(kSampT) void k_row_bins(RowScratch *__restrict__ rs
     PickBins q;
     unsigned long long a;
     q.all = S.total;
-    q.cut = crossing_bin(r, 0ull, cut_threshold(top_p), S, &q.cut_above);
+    q.cut = crossing_bin(r, 0ull, cut_threshold(top_p), S, 0, &q.cut_above);
     unsigned long long least = q.all, most = q.all;
     if (q.cut != INT32_MAX) {
         if ((int)threadIdx.x == q.cut / 4)
@@ -627,8 +635,8 @@ __global__ __launch_bounds__(kSampT) void k_row_bins(RowScratch *__restrict__ rs
         least = q.cut_above;
         most = S.total;
     }
-    q.lo = crossing_bin(r, 0ull, draw_threshold(uu, least), S, &q.lo_above);
-    q.hi = min(crossing_bin(r, 0ull, draw_threshold(uu, most), S, &a), q.cut);
+    q.lo = crossing_bin(r, 0ull, draw_threshold(uu, least), S, 1, &q.lo_above);
+    q.hi = min(crossing_bin(r, 0ull, draw_threshold(uu, most), S, 2, &a), q.cut);
     if (threadIdx.x == 0)
         R.bins = q;
 }
@@ -854,10 +862,10 @@ __global__ __launch_bounds__(kSampT) void k_row_walk(int *__restrict__ out, cons
 
 // Rows go over kSlices blocks where the rows alone leave CUs idle and are long
 // enough to pay for the launches: one block / kSlices blocks, top-p us a call,
-// 16384 entries: 50 / 39 (1 row), 51 / 64 (64 rows); 32768: 69 / 39, 75 / 69;
-// 65536: 116 / 41, 121 / 73; 128256: 183 / 44, 219 / 87 (204 / 50 at 8 rows);
-// temperature at 16384: 15 / 17, 32768: 26 / 17, 28.5 / 28.2, 128256: 89 / 30,
-// 103 / 57.  The gain shrinks with the rows: at most one row per 512 entries.
+// 32768 entries: 61 / 30 (1 row), 68 / 59 (64 rows); 65536: 104 / 32, 114 / 63;
+// 128256: 186 / 35, 204 / 76; temperature at 16384: 14 / 18, 32768: 25 / 18,
+// 27.3 / 27.7, 128256: 86 / 31, 99 / 56.  The gain shrinks with the rows: at
+// most one row per 512 entries.
 static bool long_rows(int n, int batch) { return n >= 32768 && batch <= n / 512 && batch <= 65535; }
 
 // maxima and exponentials of the rows (long_rows): p = e, not yet divided
