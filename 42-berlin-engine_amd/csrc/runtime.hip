@@ -54,6 +54,7 @@ void *workspace(size_t bytes, hipStream_t s)
     size_t want = bytes < (1u << 20) ? (1u << 20) : bytes + bytes / 4;
     if (hipMalloc(&w.ptr, want) != hipSuccess) {
         w.ptr = nullptr;
+        (void)hipGetLastError();   // reported here, and not again by the next launch's check
         set_error("workspace: hipMalloc(%zu) failed", want);
         return nullptr;
     }

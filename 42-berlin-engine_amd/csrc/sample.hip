@@ -481,7 +481,8 @@ __global__ __launch_bounds__(kSampT) void k_top_p(int *__restrict__ out, const f
 // fraction of what a CU can load, and leaves the other CUs idle; here each step
 // of the same computation is a launch of kSlices blocks per row, and after the
 // first pass only the few entries in the buckets of the two crossings are
-// looked at again (8 rows of 128256: 194 us on one block each, 42 so).  The
+// looked at again (8 rows of 128256: 194 us on one block each, 44 so, of which
+// k_row_bins 6, k_row_gather 6 and k_row_pick 16).  The
 // results are the same bits: the
 // maximum and the 62-bit sums do not depend on the order, and the sum of the
 // exponentials keeps k_probs's (block j sums, row by row of kSampT entries,
@@ -503,7 +504,9 @@ struct PickBins {
 struct alignas(16) RowScratch {
     unsigned long long hist[kSelBins];
     float pmax[kSlices], psum[kSlices];
-    int cnt[kSlices * kSlices];   // candidates found by each wave of each block
+    // candidates found by each wave of each block, their place in the row's
+    // list, and the row's
+    int cnt[kSlices * kSlices], at[kSlices * kSlices], total;
     PickBins bins;
 };
 
@@ -513,7 +516,8 @@ __device__ __forceinline__ float logit(const void *logits, size_t i)
     return BF16 ? bf16_to_f32(((const uint16_t *)logits)[i]) : ((const float *)logits)[i];
 }
 
-// the slices' maxima; clears the row's buckets for k_row_hist
+// the slices' maxima; clears the row's buckets for k_row_hist and the count of
+// its candidates for k_row_gather
 template <bool BF16>
 __global__ __launch_bounds__(kSampT) void k_row_max(RowScratch *__restrict__ rs, const void *__restrict__ logits, int n)
 {
@@ -522,6 +526,8 @@ __global__ __launch_bounds__(kSampT) void k_row_max(RowScratch *__restrict__ rs,
     RowScratch &R = rs[b];
     for (int i = blockIdx.x * (kSelBins / kSlices) + tid; i < (int)(blockIdx.x + 1) * (kSelBins / kSlices); i += kSampT)
         R.hist[i] = 0ull;
+    if (blockIdx.x == 0 && tid == 0)
+        R.total = 0;
     int c0, c1;
     slice_of(n, blockIdx.x, kSlices, kSampT, c0, c1);
     float m = -INFINITY;
@@ -642,7 +648,10 @@ __global__ __launch_bounds__(kSampT) void k_row_bins(RowScratch *__restrict__ rs
 }
 
 // Each wave lists the entries of those buckets in its slice, in ascending
-// order, as (bits << 32 | index) from the slice's own place in `cand` on.
+// order, as (bits << 32 | index), in a run of the row's list that it claims
+// after it has counted them.  The list holds kCandMax entries, as many as
+// k_row_pick takes: past that nothing is written.
+constexpr int kCandMax = 4096;
 __global__ __launch_bounds__(kSampT) void k_row_gather(unsigned long long *__restrict__ cand,
                                                        RowScratch *__restrict__ rs, const float *__restrict__ p,
                                                        int n)
@@ -654,25 +663,39 @@ __global__ __launch_bounds__(kSampT) void k_row_gather(unsigned long long *__res
     int c0, c1, cnt = 0;
     slice_of(n, part, kSlices * kSlices, kWave, c0, c1);
     const float *pb = p + (size_t)b * n;
-    unsigned long long *cb = cand + (size_t)b * n + c0;
-    wave_steps<8, unsigned>([&](int i) { return __float_as_uint(pb[i]); }, c0, c1, [&](int a, unsigned k) {
+    auto ld = [&](int i) { return __float_as_uint(pb[i]); };
+    auto wanted = [&](int a, unsigned k) {
         const int d = kSelBins - 1 - (int)(k >> kSelShift[0]);   // negative for patterns above 1
-        const bool in = a + lane < c1 && d >= 0 && (d == cut || (d >= lo && d <= hi));
-        const unsigned long long m = __ballot(in);
-        if (in)
-            cb[cnt + __popcll(m & ((1ull << lane) - 1))] = (unsigned long long)k << 32 | (unsigned)(a + lane);
-        cnt += __popcll(m);
+        return a + lane < c1 && d >= 0 && (d == cut || (d >= lo && d <= hi));
+    };
+    wave_steps<8, unsigned>(ld, c0, c1, [&](int a, unsigned k) {
+        cnt += __popcll(__ballot(wanted(a, k)));
         return false;
     });
-    if (lane == 0)
+    int at = 0;
+    if (lane == 0) {
+        at = cnt ? atomicAdd(&R.total, cnt) : 0;
         R.cnt[part] = cnt;
+        R.at[part] = at;
+    }
+    at = __builtin_amdgcn_readfirstlane(at);
+    if (cnt == 0 || at + cnt > kCandMax)
+        return;
+    unsigned long long *cb = cand + (size_t)b * kCandMax + at;
+    wave_steps<8, unsigned>(ld, c0, c1, [&](int a, unsigned k) {
+        const bool in = wanted(a, k);
+        const unsigned long long m = __ballot(in);
+        if (in)
+            cb[__popcll(m & ((1ull << lane) - 1))] = (unsigned long long)k << 32 | (unsigned)(a + lane);
+        cb += __popcll(m);
+        return false;
+    });
 }
 
 // The draw over the listed entries, one block per row: few enough for LDS, and
 // a small block, whose many barriers are cheap.  Where they are too many
 // (equal or nearly equal logits) the passes read the whole row instead.
 constexpr int kPickT = 512;
-constexpr int kCandMax = 4096;
 struct TopPPick : SelShared<1 << kSelBits[1]> {
     alignas(16) int start[kSlices * kSlices];
 };
@@ -689,10 +712,11 @@ __global__ __launch_bounds__(kPickT) void k_row_pick(int *__restrict__ out, cons
     const PickBins q = R.bins;
     const float uu = u[b];
     const float *pb = p + (size_t)b * n;
-    const unsigned long long *cb = cand + (size_t)b * n;
+    const unsigned long long *cb = cand + (size_t)b * kCandMax;
     // the parts' places in the list; a wave copies parts wave, wave + NW, ...
-    int total = 0;
-    {
+    const int total = R.total;
+    const bool listed = total <= kCandMax;
+    if (wave == 0) {
         const int4 c = *(const int4 *)&R.cnt[4 * lane];
         int v = c.x + c.y + c.z + c.w, incl = v;
 #pragma unroll
@@ -700,19 +724,16 @@ __global__ __launch_bounds__(kPickT) void k_row_pick(int *__restrict__ out, cons
             const int a = __shfl_up(incl, o, kWave);
             incl += lane >= o ? a : 0;
         }
-        total = __builtin_amdgcn_readlane(incl, kWave - 1);
-        if (wave == 0)
-            *(int4 *)&S.start[4 * lane] = make_int4(incl - v, incl - v + c.x, incl - v + c.x + c.y, incl - c.w);
+        *(int4 *)&S.start[4 * lane] = make_int4(incl - v, incl - v + c.x, incl - v + c.x + c.y, incl - c.w);
     }
     __syncthreads();
-    const bool listed = total <= kCandMax;
     if (listed)
         for (int i0 = wave; i0 < parts; i0 += NW * 8) {
             unsigned long long c[8];
-            int cnt[8], c0[8], c1;
+            int cnt[8], c0[8];
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                slice_of(n, i0 + NW * j, parts, kWave, c0[j], c1);
+                c0[j] = R.at[i0 + NW * j];
                 cnt[j] = R.cnt[i0 + NW * j];
                 c[j] = lane < cnt[j] ? cb[c0[j] + lane] : 0ull;
             }
@@ -862,10 +883,12 @@ __global__ __launch_bounds__(kSampT) void k_row_walk(int *__restrict__ out, cons
 
 // Rows go over kSlices blocks where the rows alone leave CUs idle and are long
 // enough to pay for the launches: one block / kSlices blocks, top-p us a call,
-// 32768 entries: 61 / 30 (1 row), 68 / 59 (64 rows); 65536: 104 / 32, 114 / 63;
-// 128256: 186 / 35, 204 / 76; temperature at 16384: 14 / 18, 32768: 25 / 18,
-// 27.3 / 27.7, 128256: 86 / 31, 99 / 56.  The gain shrinks with the rows: at
-// most one row per 512 entries.
+// 16384 entries: 41 / 31 (1 row), 44 / 37 (16 rows), 45 / 54 (64); 32768: 61 / 33
+// (1 row), 68 / 58 (64 rows); 65536: 104 / 35, 114 / 64; 128256: 186 / 38, 204 / 77
+// (277 / 190 at 250 rows); temperature at 16384: 14 / 18, 32768: 25 / 18, 27.3 /
+// 27.7, 128256: 86 / 31, 99 / 56.  One line for both, where no row count loses
+// yet: it is temperature's, and top-p's for few rows lies lower.  The gain
+// shrinks with the rows: at most one row per 512 entries.
 static bool long_rows(int n, int batch) { return n >= 32768 && batch <= n / 512 && batch <= 65535; }
 
 // maxima and exponentials of the rows (long_rows): p = e, not yet divided
@@ -906,12 +929,10 @@ extern "C" int be42_sample_temperature_dt(int *out, const void *logits, int logi
     BE42_CHECK(out && logits && r, "be42_sample_temperature: null pointer");
     BE42_CHECK(n > 0 && batch > 0, "be42_sample_temperature: n %d, batch %d", n, batch);
     hipStream_t s = as_stream(stream);
-    if (long_rows(n, batch)) {
-        const size_t rsb = sizeof(RowScratch) * (size_t)batch, pb = (size_t)n * batch * 4;
-        const size_t per = (size_t)(n + kWave - 1) / kWave + kSlices;
-        uint8_t *ws = (uint8_t *)workspace(rsb + pb + per * batch * 4, s);
-        if (!ws)
-            return BE42_ENOMEM;
+    const size_t rsb = sizeof(RowScratch) * (size_t)batch, pb = (size_t)n * batch * 4;
+    const size_t per = (size_t)(n + kWave - 1) / kWave + kSlices;
+    // without the memory: one block per row, which needs pb
+    if (uint8_t *ws = long_rows(n, batch) ? (uint8_t *)workspace(rsb + pb + per * batch * 4, s) : nullptr) {
         RowScratch *rs = (RowScratch *)ws;
         float *p = (float *)(ws + rsb), *steps = (float *)(ws + rsb + pb);
         const int rc = row_exp_launch(p, rs, logits, logits_bf16 != 0, n, batch, temp, false, s);
@@ -922,7 +943,7 @@ extern "C" int be42_sample_temperature_dt(int *out, const void *logits, int logi
         BE42_LAUNCH_CHECK();
         return BE42_OK;
     }
-    float *p = (float *)workspace((size_t)n * batch * 4, s);
+    float *p = (float *)workspace(pb, s);
     if (!p)
         return BE42_ENOMEM;
     const int rc = probs_launch(p, logits, logits_bf16 != 0, n, batch, temp, false, s);
@@ -945,11 +966,9 @@ extern "C" int be42_sample_top_p_dt(int *out, const void *logits, int logits_bf1
     BE42_CHECK(out && logits && u, "be42_sample_top_p: null pointer");
     BE42_CHECK(n > 0 && batch > 0, "be42_sample_top_p: n %d, batch %d", n, batch);
     hipStream_t s = as_stream(stream);
-    if (long_rows(n, batch)) {
-        const size_t rsb = sizeof(RowScratch) * (size_t)batch, cb = (size_t)n * batch * 8;
-        uint8_t *ws = (uint8_t *)workspace(rsb + cb + cb / 2, s);
-        if (!ws)
-            return BE42_ENOMEM;
+    const size_t rsb = sizeof(RowScratch) * (size_t)batch, cb = (size_t)kCandMax * batch * 8, pb = (size_t)n * batch * 4;
+    // without the memory: one block per row, which needs pb
+    if (uint8_t *ws = long_rows(n, batch) ? (uint8_t *)workspace(rsb + cb + pb, s) : nullptr) {
         RowScratch *rs = (RowScratch *)ws;
         unsigned long long *cand = (unsigned long long *)(ws + rsb);
         float *p = (float *)(ws + rsb + cb);
@@ -964,7 +983,7 @@ extern "C" int be42_sample_top_p_dt(int *out, const void *logits, int logits_bf1
         BE42_LAUNCH_CHECK();
         return BE42_OK;
     }
-    float *p = (float *)workspace((size_t)n * batch * 4, s);
+    float *p = (float *)workspace(pb, s);
     if (!p)
         return BE42_ENOMEM;
     const int rc = probs_launch(p, logits, logits_bf16 != 0, n, batch, temp, true, s);

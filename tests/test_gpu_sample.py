@@ -232,3 +232,21 @@ def test_rows_over_several_blocks(be, n, kind):
                 assert torch.equal(got, want[:4]), (u, dt, top_p)
             got, want = be.sample_temperature(a, 0.8, ut), be.sample_temperature(m, 0.8, um)
             assert torch.equal(got, want[:4]), (u, dt)
+
+
+def test_top_p_workspace(be):
+    """250 rows of 128256 equal logits (every entry is a candidate of both
+    cuts) take 4 bytes an entry and at most 80 KB a row of device memory, with
+    the workspace's growth of a quarter; an entry's 12 bytes would be 480 MB.
+    The picks are those of the rows one at a time."""
+    n, B = 128256, 250
+    x = torch.zeros((B, n), device="cuda")
+    u = torch.linspace(0, 1, B, device="cuda")
+    one = torch.cat([be.sample_top_p(x[b:b + 1], 0.8, 0.9, u[b:b + 1]) for b in (0, 100, 249)])
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    got = be.sample_top_p(x, 0.8, 0.9, u)
+    torch.cuda.synchronize()
+    taken = free - torch.cuda.mem_get_info()[0]
+    assert taken <= 1.25 * B * (4 * n + 80 * 1024) + (32 << 20), taken
+    assert torch.equal(got[[0, 100, 249]], one)
