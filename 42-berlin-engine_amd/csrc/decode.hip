@@ -1436,6 +1436,10 @@ extern "C" int be42_decoder_create(be42_decoder **out, const be42_decoder_config
             d->fail_barriers = fb && fb[0] == '1';
         }
     }
+    // the fills above are the null stream's; steps run on gstream, which does
+    // not wait for it, and take any exchange word that is not kFEmpty for a value
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(nullptr);
     if (e == hipSuccess)
         d->next_host[kMaxBatch] = 0;
     if (e != hipSuccess) {

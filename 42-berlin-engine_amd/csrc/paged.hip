@@ -289,6 +289,9 @@ extern "C" int be42_kv_create(be42_kv_pool **out, int kind, int n_layers, int n_
         e = hipMemcpy((void *)P.hpT, hpT_host, head_dim * 16 * sizeof(float), hipMemcpyHostToDevice);
     else if (e == hipSuccess)
         e = hipMemset((void *)P.hpT, 0, head_dim * 16 * sizeof(float));
+    // the fills are the null stream's, which the pool's callers need not wait for
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
         be42_kv_destroy(&P);
         return hip_fail(e, "be42_kv_create", __FILE__, __LINE__);

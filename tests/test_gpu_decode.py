@@ -14,6 +14,9 @@ step computed (captured per layer), so both caches hold the same codes, and
 every step must agree within the north star's 1e-3 (measured ~1e-6).  A step
 whose oracle top-2 logits are closer than 1e-4 relative is a near tie, where a
 different argmax is allowed and the comparison of that sequence ends."""
+import contextlib
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -409,3 +412,71 @@ def test_barrier_timeout_is_reported(be, orc, monkeypatch):
     ok.status()
     assert ok.step([2], 1).shape == (1,)
     ok.close()
+
+
+@contextlib.contextmanager
+def busy_default_stream():
+    """Keeps a few one-wave spin kernels (a million clocks each) queued on the
+    default stream from another thread, so that whatever is queued there runs
+    late while the CUs stay free."""
+    stop, full = threading.Event(), threading.Event()
+
+    def work():
+        torch.cuda.set_device(0)
+        queued = []
+        while not stop.is_set():
+            torch.cuda._sleep(1_000_000)
+            queued.append(torch.cuda.Event())
+            queued[-1].record(torch.cuda.default_stream())
+            if len(queued) > 8:
+                full.set()
+                queued.pop(0).synchronize()
+        torch.cuda.synchronize()
+
+    t = threading.Thread(target=work)
+    t.start()
+    assert full.wait(60)
+    try:
+        yield
+    finally:
+        stop.set()
+        t.join()
+
+
+def test_created_while_default_stream_is_busy(be, orc):
+    """A decoder and a page pool are ready when their creation returns: used at
+    once on a stream that does not wait for the default stream, while that is
+    busy, they give what they give on an idle GPU (their buffers are filled on
+    the default stream)."""
+    rng = np.random.default_rng(11)
+    w = make_model(rng, 3, 512, 8, 8, 64, 1408, 512, "int8")
+    _, gc = configs(3, 512, 8, 8, 64, 1408, 512, 64, 1, "int8", OR_KV_BF16, 8, 64)
+    _, hpT = orc.lsh_init(64, 42)
+    wd = to_device(w)
+    k, v = torch.randn(40, 8 * 64, device="cuda"), torch.randn(40, 8 * 64, device="cuda")
+    q = torch.randn(1, 8, 64, device="cuda")
+    side = torch.cuda.Stream()
+
+    def run():
+        with torch.cuda.stream(side):
+            dec, out = be42.Decoder(be, gc, wd, hpT), []
+            for pos in range(3):
+                lg = torch.full((1, 512), float("nan"), device="cuda")
+                dec.step([5 + pos], pos, logits=lg, sync=False)
+                out.append(lg)
+            pool = be.kv_pool(OR_KV_BF16, 1, 8, 64, 4)
+            pool.append(0, k, v, 0)
+            out.append(be.lsh_attention(pool, q, 64, 64, 0.125, want_sel=False)[0])
+            side.synchronize()
+        dec.status()
+        got = [o.cpu().numpy() for o in out]
+        dec.close()
+        pool.close()
+        return got
+
+    torch.cuda.synchronize()
+    want = run()
+    with busy_default_stream():
+        got = run()
+    for g, w_ in zip(got, want):
+        np.testing.assert_array_equal(g, w_)
