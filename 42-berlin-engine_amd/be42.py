@@ -544,7 +544,7 @@ class Decoder:
         return int(nxt[0])
 
     def status(self):
-        """Waits for the queued steps; raises if a grid barrier timed out."""
+        """Waits for the queued steps; raises if a wait of theirs gave up."""
         self.lib._call("be42_decoder_status", self.handle)
 
     def capture(self, q=None, nsel=None):

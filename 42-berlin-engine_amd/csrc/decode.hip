@@ -489,7 +489,7 @@ __device__ __forceinline__ void lds_barrier()
 struct ExWait {
     int *err;
     unsigned spin_max;   // polls before a wait gives up
-    bool never;          // a test: no wait completes
+    unsigned never;      // a test: bit w: no vector of wave w arrives; all bits: no wait completes
 };
 // after `spins` polls of a wait: whether to give up (the bound is reached, or
 // another wait of the launch has given up)
@@ -532,7 +532,7 @@ __device__ __forceinline__ void vec_to_lds(const float *src, float *dst, int n, 
         unsigned left = 0;
 #pragma unroll 2
         for (int q = 0; q < nq; q++) {
-            bool empty = wt.never;
+            bool empty = wt.never >> wave & 1;
             if (lane < left4 - q * kRowT) {
                 const uint4 u = *(const uint4 *)(dw + 4 * (lane + q * kRowT));
                 empty |= max(max(u.x, u.y), max(u.z, u.w)) == kFEmpty;
@@ -827,12 +827,14 @@ __device__ __forceinline__ float *dig_stage(uint8_t *dig, int nd, int K)
 // Waves 0-3 of a block wait for each other through an LDS counter (waves
 // 4-7 take no part: they may be stalled issuing weight loads, and a block
 // barrier would hold waves 0-3 behind them).  Every call adds 4 to the
-// target; the wait is bounded like the exchange's.  The four waves are at most a
-// few hundred cycles apart: they poll without sleeping (3B step 2024 -> 2015 us).
+// target.  A phase's first meeting can last as long as the slowest of the four
+// waits for its part of the vector.  It needs no bound of its own: the others
+// come when their waits in vec_to_lds end, which are bounded and depend on no
+// wave that waits here, so a vector that never comes is reported there.  They
+// poll without sleeping (3B step 2024 -> 2015 us).
 struct QuadSync {
     int *cnt;     // LDS, 0 at kernel start
     int target;
-    int *err;     // the launch's error flag
 };
 __device__ __forceinline__ void quad_sync(QuadSync &q)
 {
@@ -840,14 +842,8 @@ __device__ __forceinline__ void quad_sync(QuadSync &q)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if ((threadIdx.x & 63) == 0)
         __hip_atomic_fetch_add(q.cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    unsigned spins = 0;
-    while (__hip_atomic_load(q.cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < q.target) {
-        if (++spins > kFSpinMax * 64) {
-            if ((threadIdx.x & 63) == 0)
-                atomicExch(q.err, 3);
-            break;
-        }
-    }
+    while (__hip_atomic_load(q.cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < q.target)
+        ;
     asm volatile("" ::: "memory");
 }
 
@@ -1071,7 +1067,7 @@ __global__ __launch_bounds__(kFT, 1) void k_fused_layer(const FusedArgs A)
         qcnt = 0;
     __syncthreads();
     const ExWait wt = A.wait;
-    QuadSync quad{&qcnt, 0, wt.err};
+    QuadSync quad{&qcnt, 0};
     v8i fr[kFMaxU];
 #pragma unroll
     for (int u = 0; u < kFMaxU; u++)
@@ -1149,7 +1145,7 @@ __global__ __launch_bounds__(kFT, 1) void k_fused_layer(const FusedArgs A)
                            : i < (G + 1) * hd ? A.ex_k + (size_t)b * hd + (i - G * hd)
                                               : A.ex_v + (size_t)b * hd + (i - (G + 1) * hd);
         float y = ld_dev(src);
-        for (unsigned spins = 1; __float_as_uint(y) == kFEmpty || wt.never; spins++) {
+        for (unsigned spins = 1; __float_as_uint(y) == kFEmpty || wt.never == ~0u; spins++) {
             if (ex_give_up(wt, spins))
                 break;
             y = ld_dev(src);
@@ -1242,7 +1238,7 @@ struct be42_decoder {
     // the fused layer of one-sequence steps: grid = the CU count; exchange
     // buffers (FusedEx) and the second residual buffer
     bool fused = false;
-    bool fail_barriers = false;   // test: every wait of the fused launches gives up
+    ExWait wait{};                // of the fused launches (a test's: some or all give up)
     int fnb = 0;
     float *fex = nullptr;
     bool fex_dirty = false;       // a step ended half-way through its launches: empty fex before the next
@@ -1432,8 +1428,14 @@ extern "C" int be42_decoder_create(be42_decoder **out, const be42_decoder_config
             if (e == hipSuccess)
                 e = hipMemset(d->fex, 0xFF, fx.x_at() * 4);   // kFEmpty
             d->fused = e == hipSuccess;
+            // a test: 1 lets no wait complete, 2 no vector of wave 0's arrive,
+            // whose wait then gives up much later than usual
             const char *fb = getenv("BE42_DECODE_FAIL_BARRIERS");
-            d->fail_barriers = fb && fb[0] == '1';
+            d->wait = ExWait{d->next + kMaxBatch, kFSpinMax, 0};
+            if (fb && fb[0] == '1')
+                d->wait = ExWait{d->next + kMaxBatch, 64, ~0u};
+            else if (fb && fb[0] == '2')
+                d->wait = ExWait{d->next + kMaxBatch, kFSpinMax * 32, 1};
         }
     }
     // the fills above are the null stream's; steps run on gstream, which does
@@ -1631,7 +1633,7 @@ static int launch_fused_layer(be42_decoder *d, int l, const AppendStepArgs *app,
     A.H = c.n_heads;
     A.KV = c.n_kv_heads;
     A.eps = c.norm_eps;
-    A.wait = ExWait{d->next + kMaxBatch, d->fail_barriers ? 64u : kFSpinMax, d->fail_barriers};
+    A.wait = d->wait;
     A.att_out = last ? nullptr : att_out;
     A.att_scale = att_scale;
     A.er = EmbRow{(const uint8_t *)d->w.emb, d->w.emb_s, start_tok};
@@ -1846,8 +1848,8 @@ static int fault_check(be42_decoder *d, bool wait, const char *what)
         }
     }
     BE42_CHECK(d->fault == 0,
-               "%s: a bounded wait gave up in an earlier step (code %d: 1 a grid barrier of the fused layer, 3 its "
-               "wave sync, 4 the split attention's); the decoder's results and cache are invalid (destroy it)",
+               "%s: a bounded wait gave up in an earlier step (code %d: 1 an exchange of the fused layer, 4 the split "
+               "attention's); the decoder's results and cache are invalid (destroy it)",
                what, d->fault);
     return BE42_OK;
 }

@@ -340,8 +340,8 @@ be42_kv_pool *be42_decoder_pool(be42_decoder *d);
  * as a HIP graph (environment BE42_DECODE_NO_GRAPH=1 launches them one by one).
  * The call returns once the host side of the step is queued; it blocks only
  * for next_tokens, or when the step before the last still runs.
- * One-sequence steps run each layer as one launch whose blocks meet at grid
- * barriers; a barrier wait that does not complete within its bound sets a
+ * One-sequence steps run each layer as one launch whose blocks exchange
+ * vectors; a wait for one that does not complete within its bound sets a
  * device flag.  The step that sets it is reported by itself when next_tokens
  * is given, else by the next be42_decoder_step / be42_decoder_prefill that
  * finds it finished, or by be42_decoder_status; from then on the decoder
@@ -349,8 +349,8 @@ be42_kv_pool *be42_decoder_pool(be42_decoder *d);
 int  be42_decoder_step(be42_decoder *d, const int *tokens, int batch, int pos, int *next_tokens,
                        float *logits_out, void *stream);
 int  be42_decoder_next_tokens(be42_decoder *d, const int **dev_ptr);
-/* Waits for the decoder's queued work; BE42_OK, or an error when a grid
- * barrier of any step so far timed out. */
+/* Waits for the decoder's queued work; BE42_OK, or an error when a
+ * bounded wait of any step so far gave up. */
 int  be42_decoder_status(be42_decoder *d);
 /* Batched prefill (forward_prefill_batch, src/inference/inference.c:718-1112,
  * with its token-major / feature-major layout fixed): the n prompt tokens of

@@ -382,11 +382,13 @@ def test_fused_layer_passes_nan_on(be, orc, monkeypatch, name):
     np.testing.assert_array_equal(run(), want)
 
 
-def test_barrier_timeout_is_reported(be, orc, monkeypatch):
-    """A fused-layer grid barrier whose wait gives up must be reported even
-    when no step asks for its tokens.  BE42_DECODE_FAIL_BARRIERS=1 makes every
-    wait of the fused launches look for a barrier number no block writes,
-    with a 64-poll bound: each wait ends, the launch runs to its end, and the
+@pytest.mark.parametrize("fail", ["1", "2"])
+def test_barrier_timeout_is_reported(be, orc, monkeypatch, fail):
+    """A fused-layer exchange whose wait gives up must be reported, as that
+    wait, even when no step asks for its tokens.  BE42_DECODE_FAIL_BARRIERS=1
+    lets no wait of the fused launches complete, with a 64-poll bound; 2 no
+    vector of wave 0's, with 32 times the usual bound, while waves 1-3 of its
+    block wait for it.  Each wait ends, the launch runs to its end, and the
     flag is set.  Steps without next_tokens are queued; the next step call
     (or be42_decoder_status) must refuse, and keep refusing."""
     rng = np.random.default_rng(5)
@@ -394,16 +396,16 @@ def test_barrier_timeout_is_reported(be, orc, monkeypatch):
     _, gc = configs(2, 512, 8, 8, 64, 1408, 4096, 256, 1, "int8", OR_KV_INT8, 8, 64)
     _, hpT = orc.lsh_init(64, 42)
     wd = to_device(w)
-    monkeypatch.setenv("BE42_DECODE_FAIL_BARRIERS", "1")
+    monkeypatch.setenv("BE42_DECODE_FAIL_BARRIERS", fail)
     dec = be42.Decoder(be, gc, wd, hpT)
     monkeypatch.delenv("BE42_DECODE_FAIL_BARRIERS")
     dec.step([1], 0, sync=False)
     torch.cuda.synchronize()
-    with pytest.raises(be42.Be42Error, match="grid barrier"):
+    with pytest.raises(be42.Be42Error, match="code 1: 1 an exchange"):
         dec.step([2], 1, sync=False)
-    with pytest.raises(be42.Be42Error, match="grid barrier"):
+    with pytest.raises(be42.Be42Error, match="code 1: 1 an exchange"):
         dec.status()
-    with pytest.raises(be42.Be42Error, match="grid barrier"):
+    with pytest.raises(be42.Be42Error, match="code 1: 1 an exchange"):
         dec.step([2], 1)
     dec.close()
     # a decoder made without the knob is unaffected
