@@ -458,7 +458,7 @@ constexpr int kFMaxU = 12;                // MFMA steps (128 k-bytes) one wave h
 constexpr int kFMaxTiles = 8;             // 16-row tiles of one block in one phase
 constexpr int kFDigBytes = 84 * 1024;     // LDS digit planes; also keeps one block per CU
 constexpr int kFWeightWait = 40;          // s_sleep units before waves 4-7 issue weight loads behind an exchange
-constexpr unsigned kFSpinMax = 1u << 16;  // polls (about 1 us each) before a wait gives up
+constexpr unsigned kFSpinMax = 1u << 18;  // polls (0.3 us each, 1 - 3 behind other loads: at least 80 ms) before a wait gives up
 
 __device__ __forceinline__ float ld_dev(const float *p)
 {
@@ -1435,7 +1435,7 @@ extern "C" int be42_decoder_create(be42_decoder **out, const be42_decoder_config
             if (fb && fb[0] == '1')
                 d->wait = ExWait{d->next + kMaxBatch, 64, ~0u};
             else if (fb && fb[0] == '2')
-                d->wait = ExWait{d->next + kMaxBatch, kFSpinMax * 32, 1};
+                d->wait = ExWait{d->next + kMaxBatch, kFSpinMax * 8, 1};
         }
     }
     // the fills above are the null stream's; steps run on gstream, which does

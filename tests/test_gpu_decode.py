@@ -16,6 +16,7 @@ whose oracle top-2 logits are closer than 1e-4 relative is a near tie, where a
 different argmax is allowed and the comparison of that sequence ends."""
 import contextlib
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -387,7 +388,7 @@ def test_barrier_timeout_is_reported(be, orc, monkeypatch, fail):
     """A fused-layer exchange whose wait gives up must be reported, as that
     wait, even when no step asks for its tokens.  BE42_DECODE_FAIL_BARRIERS=1
     lets no wait of the fused launches complete, with a 64-poll bound; 2 no
-    vector of wave 0's, with 32 times the usual bound, while waves 1-3 of its
+    vector of wave 0's, with eight times the usual bound, while waves 1-3 of its
     block wait for it.  Each wait ends, the launch runs to its end, and the
     flag is set.  Steps without next_tokens are queued; the next step call
     (or be42_decoder_status) must refuse, and keep refusing."""
@@ -399,8 +400,14 @@ def test_barrier_timeout_is_reported(be, orc, monkeypatch, fail):
     monkeypatch.setenv("BE42_DECODE_FAIL_BARRIERS", fail)
     dec = be42.Decoder(be, gc, wd, hpT)
     monkeypatch.delenv("BE42_DECODE_FAIL_BARRIERS")
+    torch.cuda.synchronize()
+    start = time.monotonic()
     dec.step([1], 0, sync=False)
     torch.cuda.synchronize()
+    if fail == "2":
+        # a usual bound of 50 ms at least: blocks of the launch may wait that
+        # long for CUs that another stream's kernels hold
+        assert time.monotonic() - start >= 8 * 0.05
     with pytest.raises(be42.Be42Error, match="code 1: 1 an exchange"):
         dec.step([2], 1, sync=False)
     with pytest.raises(be42.Be42Error, match="code 1: 1 an exchange"):
