@@ -2,8 +2,9 @@
 device scratch (no allocation), called through the C ABI, against the
 allocating entry point (be42_gemv_q8 / be42_gemv_fp8) on the same inputs --
 the same kernels, so the outputs must be bit-identical -- and against the
-oracle within the north star's 1e-3.  Two calls in a row share the scratch,
-the second with a smaller input; a shape past the scratch is refused."""
+oracle within the north star's 1e-3.  Calls in a row share the scratch,
+later ones with smaller inputs of another k, batch and digit layout, or form
+their digits in the one launch without it; a shape past the scratch is refused."""
 import ctypes as C
 
 import numpy as np
@@ -31,8 +32,10 @@ def _noalloc(be, y, w, s, x, n, k, b, kind):
 @pytest.mark.parametrize("kind", ["int8", "fp8"])
 def test_gemv_noalloc_matches_gemv(be, orc, kind):
     rng = np.random.default_rng(77 if kind == "int8" else 78)
-    # a split-K launch (4096 x 14336 at batch 16), then a smaller one
-    for n, k, b in ((4096, 14336, 16), (300, 1024, 3)):
+    # a split-K launch (4096 x 14336 at batch 16), then smaller ones: more digit
+    # columns than the one-launch GEMV takes, a longer row than it takes, and
+    # one that it takes (no scratch)
+    for n, k, b in ((4096, 14336, 16), (300, 1024, 8), (100, 8192, 1), (300, 1024, 3)):
         wq, ws = _weights(rng, kind, n, k)
         x = rng.standard_normal((b, k)).astype(np.float32)
         wt, st, xt = torch.from_numpy(wq).cuda(), torch.from_numpy(ws).cuda(), torch.from_numpy(x).cuda()
