@@ -582,7 +582,7 @@ struct FusedArgs {
     const AppendStepArgs *app;              // the next layer's append
     const float *cos_t, *sin_t;
     const int *pos_p;
-    int rope_len, dim, hidden, qd, kd, H, KV;
+    int rope_len, dim, H, KV;
     float eps;
     ExWait wait;
     float *att_out;      // the next layer's dense attention output (null: a launch of its own)
@@ -661,17 +661,15 @@ __device__ __forceinline__ FWave ph_wave(int nt, int steps, int wave)
     return w;
 }
 
-// this wave's weight fragments of the phase (waves lo .. hi-1 only): lane
+// this wave's weight fragments of the phase: lane
 // (r, g) holds row r of its tile, k bytes 128 s + 16 g .. + 15 and
 // 128 s + 64 + 16 g .. + 15 of each of its steps s (so each load instruction
 // reads 64 contiguous bytes of each of 16 rows; the digit fragments use the
 // same k positions)
-__device__ __forceinline__ void ph_prefetch(const FPhase &ph, int b, int nb, v8i (&fr)[kFMaxU], int lo, int hi)
+__device__ __forceinline__ void ph_prefetch(const FPhase &ph, int b, int nb, v8i (&fr)[kFMaxU])
 {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, g = lane >> 4;
-    if (wave < lo || wave >= hi)
-        return;
     const FWave fw = ph_wave(ph_count(ph, b, nb), ph.steps, wave);
     if (!fw.on)
         return;
@@ -1090,8 +1088,11 @@ __global__ __launch_bounds__(kFT, 1) void k_fused_layer(const FusedArgs A)
             lds_barrier();
             // The weight loads fill the CU's memory queue for 1.5 - 3 us, and a
             // poll behind them waits as long: leave the queue to the polls for
-            // about as long as the vector takes to arrive.  3B step by the sleep
-            // (64 cycles each): 0 1970 us, 12 1946, 24 1947, 40 1924, 80 1992.
+            // about as long as the vector takes to arrive.  Dense steps of one
+            // sequence by the sleep (64 cycles each: 0 / 12 / 24 / 40 / 80), us: 4
+            // layers of 512 floats 170 / 170 / 169 / 169 / 178, 8 of 1024 330 / 327 /
+            // 327 / 330 / 344, 8 of 2048 443 / 436 / 434 / 438 / 451, the 3B model
+            // 1751 / 1735 / 1733 / 1716 / 1789.
             if (p > 0)
                 __builtin_amdgcn_s_sleep(kFWeightWait);
         } else if (START || (p & 1)) {
@@ -1107,7 +1108,7 @@ __global__ __launch_bounds__(kFT, 1) void k_fused_layer(const FusedArgs A)
             vec_digits<FP8>(p == 0 ? A.att : A.ex_h2, ph.K, p != 0, dig, red, quad, wt, [] { lds_barrier(); });
         }
         asm volatile("" ::: "memory");
-        ph_prefetch(ph, b, nb, fr, 0, kFW);
+        ph_prefetch(ph, b, nb, fr);
         lds_barrier();
         ph_compute<FP8>(ph, b, nb, fr, dig, ph.K, red[12], part, ybuf, oo);
         if (p == A.last)
@@ -1285,12 +1286,11 @@ static bool fused_layer_fits(const be42_decoder_config &c, be42_decoder *d)
     if (c.dim % 128 || c.hidden_dim % 128 || qd % 128 || kd % 16 || c.dim > 4096 ||
         c.hidden_dim > kRowT * 4 * kFVecG || qd > kRowT * 4 * kFVecG ||
         (size_t)(nd + 4) * std::max(c.hidden_dim, qd) + 16 > (size_t)kFDigBytes ||
-        (size_t)(nd + 8) * c.dim + 16 > (size_t)kFDigBytes ||
+        (size_t)(nd + 4) * c.dim + 16 > (size_t)kFDigBytes ||
         (size_t)(c.n_heads / c.n_kv_heads + 2) * c.head_dim * 4 + 1024 > (size_t)kFDigBytes || c.n_kv_heads > cus)
         return false;
     // one block per CU, but no more blocks than the largest phase has row
-    // tiles (or gate/up tile pairs): a small model's barriers then gather
-    // fewer blocks
+    // tiles (or gate/up tile pairs): a block without tiles would only poll
     const int units_max = std::max(std::max((c.dim + 15) / 16, (c.hidden_dim + 15) / 16),
                                    (qd + 2 * kd + 15) / 16 + 2);
     const int nb = std::max(std::min(cus, units_max), c.n_kv_heads);
@@ -1627,9 +1627,6 @@ static int launch_fused_layer(be42_decoder *d, int l, const AppendStepArgs *app,
     A.pos_p = pos_p;
     A.rope_len = rope_len;
     A.dim = dim;
-    A.hidden = hidden;
-    A.qd = qd;
-    A.kd = kd;
     A.H = c.n_heads;
     A.KV = c.n_kv_heads;
     A.eps = c.norm_eps;
