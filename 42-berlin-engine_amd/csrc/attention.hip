@@ -1414,10 +1414,8 @@ int lsh_attention_digits(const be42_kv_pool &P, const float *q, const int *slots
                            s);
 }
 
-// The router runs once per query (k_route), then the attention of every
-// (query, KV head) pair over that selection (k_attn_fused at 16 waves, the
-// layout a one-query decode launch sums in); k_lsh_attn would repeat the
-// router in each KV head's workgroup.
+// T consecutive tokens from pos0 on, each of which sees at most kFusedMaxPages
+// pages and attends to all of them (k_attn_prompt; H / n_kv 1 .. 4).
 template <int HD>
 static int launch_prompt(const be42_kv_pool &P, const float *q, int slot, int pos0, int T, int H, float scale,
                          float *out, hipStream_t s)
@@ -1440,6 +1438,11 @@ static int launch_prompt(const be42_kv_pool &P, const float *q, int slot, int po
     }
 }
 
+// The tokens that attend to every page go together where they are many
+// (launch_prompt).  For the others the router runs once per query (k_route),
+// then the attention of every (query, KV head) pair over that selection
+// (k_attn_fused at 16 waves, the layout a one-query decode launch sums in);
+// k_lsh_attn would repeat the router in each KV head's workgroup.
 int lsh_attention_prefix(const be42_kv_pool &P, const float *q, int slot, int pos0, const int *slots, const int *lim,
                          int n_queries, int n_heads, int k_sel, int cand_cap, float scale, float *out, int *sel,
                          int *nsel, int sel_stride, hipStream_t s)

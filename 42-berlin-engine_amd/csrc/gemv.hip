@@ -1363,8 +1363,8 @@ static void launch_cfg(const GemvSegs &S, const uint8_t *dig, const float *sx, i
 }
 
 // Launch shape per (dtype, column groups NC, rows n, k), measured on MI355X
-// over the decode projections of configs[0] and configs[4] and the four
-// configs[1] shapes at batch 1 / 4 / 8 / 16 (rows n count all segments of a
+// over the decode projections of the tiny and the 3B decoder and four shapes
+// of 4096 - 128256 rows at batch 1 / 4 / 8 / 16 (rows n count all segments of a
 // launch).  RT row tiles of 16 per wave, U MFMA steps per burst, KS waves
 // splitting K per row group, WAVES per block, PF register double buffering.
 struct TileCfg {

@@ -21,15 +21,16 @@
 //
 // Top-p never sorts: both cuts are weighted selections.  The entry at which
 // the descending-order running sum first exceeds a threshold is found by a
-// most-significant-byte-first radix select over the bit patterns of the
+// most-significant-first radix select over the bit patterns of the
 // (non-negative) probabilities, where each pass sums the probabilities of the
-// remaining candidates per byte value and keeps the byte whose bucket holds
-// the crossing; after four passes the crossing entry's value is known, and
-// among the entries of that value (ascending index) the crossing is the
-// (T - sum above) / value-th.  The sums are exact: probabilities as 62-bit
-// fixed point (p * 2^62, truncated) in 64-bit integer additions, so they do
-// not depend on the order of the atomic additions, and they are the float64
-// running sums to ~n * 2^-62 -- closer than the reference's fp32 sums.
+// remaining candidates per value of a bit field (kSelBits) and keeps the one
+// whose bucket holds the crossing; after three passes the crossing entry's
+// value is known, and among the entries of that value (ascending index) the
+// crossing is the (T - sum above) / value-th.  The sums are exact:
+// probabilities as 62-bit fixed point (p * 2^62, truncated) in 64-bit integer
+// additions, so they do not depend on the order of the atomic additions, and
+// they are the float64 running sums to ~n * 2^-62 -- closer than the
+// reference's fp32 sums.
 #include <cstring>
 
 #include "be42_common.h"
