@@ -1101,8 +1101,13 @@ static void launch_dma(const GemvSegs &S, const uint8_t *dig, const float *sx, i
 // it).  Operands and epilogue are k_gemv's (32 consecutive bytes of a row per
 // lane and step for both types, the digits read at the same k), so INT8
 // results are the same bits.
-// Latency bound: 512 x 512 INT8 batch 1 5.7 -> 3.2 us a call, 4096 x 4096 8.9 ->
-// 6.9 us (2.4 TB/s), 8192 x 4096 14.0 -> 10.1 us (3.3 TB/s).
+// The weights are plain loads: lanes that share a cache line load it at
+// different steps, and a non-temporal line is fetched again for the second
+// (FP8 batch 2, us, non-temporal / plain: 8192 x 3088 12.1 / 7.6 from the caches
+// and 12.9 / 10.0 from HBM, 8192 x 4096 10.6 / 8.4 and 11.6 / 11.4).
+// Latency bound: us a call in two launches / in one, weights in the caches and
+// from HBM: 512 x 512 INT8 batch 1 5.1 / 2.9; 4096 x 4096 7.8 / 4.7 and 9.1 / 6.5
+// (2.6 TB/s), 8192 x 4096 11.0 / 6.8 and 14.4 / 10.0 (3.4 TB/s).
 constexpr int kDirectWaves = 8;
 constexpr int kDirectX = 5;                      // float4s of x per thread: batch * KU <= 10
 constexpr int direct_row(int ku) { return ku * 1024 + 16; }   // a digit column in LDS, padded against bank conflicts
@@ -1154,8 +1159,8 @@ __global__ __launch_bounds__(kDirectWaves * 64) void k_gemv_direct(float *__rest
         const uint8_t *wr = W + (size_t)row * K;
 #pragma unroll
         for (int s = 0; s < KU; s++) {
-            w[t][s][0] = __builtin_nontemporal_load((const v4i *)(wr + min(kb + 128 * s, klast)));
-            w[t][s][1] = __builtin_nontemporal_load((const v4i *)(wr + min(kb + 128 * s + 16, klast)));
+            w[t][s][0] = *(const v4i *)(wr + min(kb + 128 * s, klast));
+            w[t][s][1] = *(const v4i *)(wr + min(kb + 128 * s + 16, klast));
         }
     }
     asm volatile("" ::: "memory");
@@ -1252,14 +1257,15 @@ static int launch_direct(float *y, const uint8_t *w, const float *sw, const floa
 
 // Whether (n, k, batch) runs as one k_gemv_direct launch; *rc its result.  The
 // lines lie where forming the digits in every block costs what the launch
-// saves (~1.3 us per 4096 elements of x; us, two launches / one, HBM-resident
-// weights, INT8, FP8 alike): 512 x 512 batch 1 5.7 / 3.2, batch 4 6.2 / 4.2;
-// 3072 x 3072 batch 1 7.7 / 5.2, batch 2 7.8 / 6.1, batch 4 8.0 / 8.2; 4096 x
-// 4096 batch 1 8.9 / 6.9, batch 2 9.1 / 8.2, batch 4 9.3 / 10.9; 8192 x 4096
-// batch 1 14.0 / 10.1; 16384 x 2048 batch 1 12.2 / 8.5, batch 5 12.6 / 12.2;
-// and where a block's weights stop fitting in 64 registers (14336 x 4096 batch
-// 1 15.4 / 16.4; 3000 x 8000 batch 1, weights in the Infinity Cache, 11.1 /
-// 11.5).
+// saves (~1.3 us per 4096 elements of x; us, two launches / one, INT8, FP8
+// alike, weights in the caches and from HBM): 512 x 512 batch 4 5.4 / 3.8 and
+// 5.5 / 3.8; 3072 x 3072 batch 1 6.8 / 4.1 and 7.8 / 4.6, batch 3 7.1 / 5.8 and
+// 8.2 / 6.4; 4096 x 4096 batch 2 8.1 / 6.4 and 9.3 / 7.9; 16384 x 2048 batch 1
+// 11.4 / 6.3 and 12.4 / 8.4, batch 5 11.3 / 10.1 and 12.8 / 12.1; 8448 x 1792
+// batch 5 9.8 / 9.6 and 10.1 / 10.3 (133 blocks); 4096 x 2000 batch 5 6.0 / 6.1
+// and 7.4 / 7.2.  Past the lines, measured with non-temporal weights from HBM:
+// 3072 x 3072 batch 4 8.0 / 8.2, 4096 x 4096 batch 4 9.3 / 10.9, and where a
+// block's weights stop fitting in 64 registers 14336 x 4096 batch 1 15.4 / 16.4.
 // Overlapping x and y need the digits formed before the first output.
 template <bool FP8>
 static bool gemv_direct(float *y, const uint8_t *w, const float *sw, const float *x, int n, int k, int batch,
