@@ -1417,8 +1417,14 @@ static TileCfg pick_tile(bool fp8, int nc, int n, int k, int batch)
     // 17.5 us; with four planes FP8 batch 16 is 4 groups, and 14336 x 4096
     // runs 29.1 -> 26.7 us here instead of on the split slab kernel).
     // INT8 at one column group past 4096 rows: 5120 x 3072 9.3 -> 7.8 us, 6144
-    // x 4096 10.9 -> 9.4 (FP8 stays: 7.5 against 8.4, 9.2 against 10.2).
-    if (n > 32768 || (n > 8192 && nc < 3) || (n > 4096 && nc >= 2 && nc <= 4) || (n > 4096 && !fp8 && nc == 1)) {
+    // x 4096 10.9 -> 9.4 (FP8 stays: 7.5 against 8.4, 9.2 against 10.2), where
+    // rows start on cache lines (its non-temporal loads fetch a shared line
+    // twice).  Weights of a model come from HBM; others / this one, batch 4, us
+    // with the digits' launch, from HBM and from the caches: 5120 x 3072 12.2 /
+    // 10.3 and 9.4 / 10.0, 6144 x 4096 14.4 / 12.1 and 11.3 / 11.1; off the lines
+    // 6144 x 3600 13.6 / 13.3 and 9.2 / 12.5.
+    if (n > 32768 || (n > 8192 && nc < 3) || (n > 4096 && nc >= 2 && nc <= 4) ||
+        (n > 4096 && !fp8 && nc == 1 && k % 128 == 0)) {
         const int steps = (int)(xdig_kp(k, fp8) / 128);
         if (steps % kCoopWaves == 0 && steps / kCoopWaves <= 4)
             return TileCfg{0, 6, 0, kCoopWaves, 0, 4, 1};
