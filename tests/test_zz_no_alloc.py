@@ -2,7 +2,7 @@
 device scratch (no allocation), called through the C ABI, against the
 allocating entry point (be42_gemv_q8 / be42_gemv_fp8) on the same inputs --
 the same kernels, so the outputs must be bit-identical -- and against the
-oracle within the north star's 1e-3.  Calls in a row share the scratch,
+oracle within 1e-3.  Calls in a row share the scratch,
 later ones with smaller inputs of another k, batch and digit layout, or form
 their digits in the one launch without it; a shape past the scratch is refused."""
 import ctypes as C
